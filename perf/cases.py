@@ -1,0 +1,339 @@
+"""The calls whose speed matters to a user of the solver, as listed and drawn cases.
+
+A program that uses this framework sorts its points into a tree, builds an H^2
+operator, builds and factorizes an H^2 preconditioner, then solves one or many
+right-hand sides with GMRES and checks the solutions with the dense product.
+Set-up runs once per geometry and is most of a one-off run; products,
+substitutions and solves run for as long as the problem is in use. The cases
+cover each of these calls from the smallest problem of the serial sweep
+(N = 2048) to N = 131072, on random cubes and spheres, FP64, FP32 and
+bfloat16-stored factors, one right-hand side and several.
+
+Points, vectors and solutions are made from the seed. Results are handed back
+in the type whose precision they carry: FP64 arrays that hold the outcome of an
+FP32 product or of FP32 / bfloat16 factors come back as FP32.
+"""
+import numpy as np
+import torch
+
+from mxc_amd import _native as N
+from mxc_amd.device import Context
+from mxc_amd.solver import H2, Problem, build_tree, csr, tree_levels
+
+DIAG, ALPHA, THETA = 1e3, 1.0, 2.0
+PREC = {"fp64": N.MXG_FP64, "fp32": N.MXG_FP32, "bf16": N.MXG_BF16}
+
+_context = None
+
+
+def context():
+    """The program's one device context."""
+    global _context
+    if _context is None:
+        _context = Context(0)
+    return _context
+
+
+def listed():
+    cube = dict(geometry="cube", kernel="laplace", leaf=256, sampling=2000)
+    ball = dict(geometry="sphere", kernel="yukawa", leaf=256, sampling=2000)
+    return [
+        # the smallest product: one vector, a few hundred microseconds of short launches
+        dict(name="matvec cube 4096 fp64", kind="matvec", n=4096, eps=1e-10, precision="fp64", nrhs=1, **cube),
+        # the inner product of mixed-precision solves: a batch of eight, bound by the near blocks
+        dict(name="matvec sphere 131072 fp32 x8", kind="matvec", n=131072, eps=1e-7, precision="fp32", nrhs=8, **ball),
+        # one application of the fixed-rank preconditioner of the CLI's default run
+        dict(name="substitution cube 20000 fp64", kind="substitution", n=20000, eps=0.0, rank=100, precision="fp64", nrhs=1,
+             **cube),
+        # the preconditioner inside mixed-precision solves: eight vectors, bfloat16-stored factors
+        dict(name="substitution sphere 131072 bf16 x8", kind="substitution", n=131072, eps=1e-6, rank=64, precision="bf16",
+             nrhs=8, **ball),
+        # factorizing the CLI's default preconditioner (ragged leaves of 312 and 313 points)
+        dict(name="factorize cube 20000 fp64", kind="factorize", n=20000, eps=0.0, rank=100, precision="fp64", nrhs=1, **cube),
+        # factorizing for mixed-precision solves at the largest size here
+        dict(name="factorize sphere 131072 bf16", kind="factorize", n=131072, eps=1e-6, rank=64, precision="bf16", nrhs=1,
+             **ball),
+        # building the accurate operator for the smallest problem of the serial sweep
+        dict(name="operator cube 2048", kind="operator", n=2048, eps=1e-10, precision="fp64", nrhs=1, **cube),
+        # building the accurate operator of the surface problem: the longest step of a run
+        dict(name="operator sphere 65536", kind="operator", n=65536, eps=1e-12, precision="fp64", nrhs=1, **ball),
+        # building and factorizing the fixed-rank preconditioner for the largest problem of the serial sweep
+        dict(name="preconditioner cube 32768 fp64", kind="preconditioner", n=32768, eps=0.0, rank=100, precision="fp64",
+             nrhs=1, **cube),
+        # one solve as the CLI does it: reference-mode GMRES, everything FP64
+        dict(name="gmres cube 8192 fp64", kind="gmres", n=8192, eps=1e-10, rank=100, precond_eps=0.0, inner_eps=0.0,
+             mode="reference", precision="fp64", nrhs=1, **cube),
+        # one batch of eight mixed-precision solves, as a serving or throughput program runs them
+        dict(name="gmres sphere 65536 mixed x8", kind="gmres", n=65536, eps=1e-12, rank=64, precond_eps=1e-6, inner_eps=1e-7,
+             mode="cgs2", precision="bf16", nrhs=8, **ball),
+        # the matrix-free check of a batch of solutions
+        dict(name="dense check sphere 65536 x8", kind="dense", n=65536, precision="fp64", nrhs=8, **ball),
+    ]
+
+
+# kind: (smallest and largest N on the cube, on the sphere)
+RANGES = {"matvec": ((2048, 24000), (4096, 131072)), "substitution": ((2048, 32768), (4096, 131072)),
+          "factorize": ((2048, 32768), (4096, 131072)), "operator": ((2048, 12000), (2048, 65536)),
+          "preconditioner": ((2048, 32768), (2048, 65536)), "gmres": ((2048, 12000), (4096, 65536)),
+          "dense": ((1000, 65536), (1000, 65536))}
+
+
+def _between(rng, lo, hi):
+    return int(round(lo * (hi / lo) ** rng.random()))
+
+
+def draw(rng):
+    kind = rng.choice(sorted(RANGES))
+    geometry = rng.choice(["cube", "sphere"])
+    n = _between(rng, *RANGES[kind][geometry == "sphere"])
+    c = dict(kind=kind, n=n, geometry=geometry, kernel="laplace" if geometry == "cube" else "yukawa",
+             leaf=rng.choice([128, 256, 256]), sampling=2000, precision="fp64", nrhs=1)
+    if kind == "dense":
+        c.update(kernel=rng.choice(["laplace", "yukawa", "gaussian"]), nrhs=rng.randint(1, 8))
+    elif kind == "operator":
+        c.update(eps=rng.choice([1e-7, 1e-10, 1e-12]))
+    elif kind == "matvec":
+        c.update(precision=rng.choice(["fp64", "fp32"]), nrhs=rng.choice([1, 1, rng.randint(2, 8)]))
+        c.update(eps=1e-7 if c["precision"] == "fp32" else 1e-10)
+    elif kind == "gmres":
+        if rng.random() < 0.5:
+            c.update(eps=1e-10, rank=100, precond_eps=0.0, inner_eps=0.0, mode="reference")
+        else:
+            c.update(eps=1e-12 if geometry == "sphere" else 1e-11, rank=64, precond_eps=1e-6, inner_eps=1e-7, mode="cgs2",
+                     precision=rng.choice(["fp64", "fp32", "bf16"]), nrhs=rng.randint(1, 8))
+    else:
+        c.update(precision=rng.choice(["fp64", "fp32", "bf16"]))
+        if rng.random() < 0.5:
+            c.update(eps=0.0, rank=rng.choice([32, 64, 100, 128]))
+        else:
+            c.update(eps=1e-6, rank=64)
+        if kind == "substitution":
+            c.update(nrhs=rng.choice([1, 1, rng.randint(2, 8)]))
+    return c
+
+
+# ---------------------------------------------------------------- inputs
+
+def _points(case, seed):
+    """3 n coordinates: uniform in the unit cube, or golden-angle points of the unit sphere under a random rotation."""
+    n, rng = case["n"], np.random.default_rng(seed)
+    if case["geometry"] == "cube":
+        return rng.random((n, 3))
+    i = np.arange(n)
+    y = 1.0 - 2.0 * i / (n - 1)
+    rad, t = np.sqrt(np.maximum(0.0, 1.0 - y * y)), i * np.pi * (3.0 - np.sqrt(5.0))
+    q, _ = np.linalg.qr(rng.standard_normal((3, 3)))
+    return np.stack([rad * np.cos(t), y, rad * np.sin(t)], axis=1) @ q.T
+
+
+def _tree_order(p, leaf):
+    """The points in tree order: every cell is sorted along its longest side and cut in the middle."""
+    p = p.copy()
+    cells = [(0, len(p))]
+    for _ in range(tree_levels(len(p), leaf)):
+        below = []
+        for a, b in cells:
+            axis = int(np.argmax((p[a:b].max(0) - p[a:b].min(0)) * 0.5 + 1e-8))
+            p[a:b] = p[a:b][np.argsort(p[a:b, axis], kind="stable")]
+            below += [(a, a + (b - a) // 2), (a + (b - a) // 2, b)]
+        cells = below
+    return p
+
+
+def _vectors(case, seed):
+    """nrhs x n on the GPU, U(-1, 1)."""
+    g = torch.Generator("cuda").manual_seed(7919 + seed)
+    return torch.rand((case["nrhs"], case["n"]), generator=g, dtype=torch.float64, device="cuda") * 2.0 - 1.0
+
+
+def _dense(kernel, p, x):
+    """x K in FP64 (x: nrhs x n, K symmetric), a block of rows at a time."""
+    n, out = len(p), torch.empty_like(x)
+    step = max(1, (1 << 27) // n)
+    for a in range(0, n, step):
+        d2 = (p[a:a + step, 0, None] - p[None, :, 0]).square_()
+        d2 += (p[a:a + step, 1, None] - p[None, :, 1]).square_()
+        d2 += (p[a:a + step, 2, None] - p[None, :, 2]).square_()
+        same = d2 == 0.0
+        if kernel == "gaussian":
+            k = torch.exp(-ALPHA * d2)
+            k[same] = 1.0001
+        else:
+            d = d2.sqrt_()
+            k = torch.exp(-ALPHA * d) / d if kernel == "yukawa" else 1.0 / d
+            k[same] = DIAG
+        out[:, a:a + step] = (k @ x.T).T
+    return out
+
+
+class Vec:
+    """A torch tensor (nrhs x n) as the device vectors (n x nrhs, column major) that the solver's calls take."""
+
+    def __init__(self, t):
+        self.t, self.ptr, self.shape = t, t.data_ptr(), (t.shape[1], t.shape[0])
+        self.nbytes = t.numel() * t.element_size()
+
+    def zero(self):
+        N.check_gpu(N.gpu().mxg_memset(context().handle, self.ptr, 0, self.nbytes))
+
+    def copy(self, other):
+        N.check_gpu(N.gpu().mxg_memcpy_d2d(context().handle, self.ptr, other.ptr, self.nbytes))
+
+
+class State:
+    pass
+
+
+def _operator(prob, case, eps):
+    return H2.operator(prob, eps, case["sampling"], case["kernel"], DIAG, ALPHA, THETA)
+
+
+def _preconditioner(prob, case, eps):
+    return H2.preconditioner(prob, case["rank"], case["sampling"], case["kernel"], DIAG, ALPHA, THETA, eps=eps)
+
+
+def prepare(case, seed):
+    s, kind = State(), case["kind"]
+    s.case = case
+    s.problem = Problem(context(), _points(case, seed).reshape(-1), case["leaf"])
+    x = _vectors(case, seed)
+    s.x, s.y = Vec(x), Vec(torch.empty_like(x))
+    if kind == "matvec":
+        s.A = _operator(s.problem, case, case["eps"])
+    elif kind in ("substitution", "factorize"):
+        s.M = _preconditioner(s.problem, case, case["eps"])
+        if kind == "substitution":
+            s.M.factorize(PREC[case["precision"]])
+    elif kind == "gmres":
+        s.A = _operator(s.problem, case, case["eps"])
+        mixed = case["mode"] == "cgs2" and case["precision"] != "fp64"
+        s.inner = _operator(s.problem, case, case["inner_eps"]) if mixed else None
+        s.M = _preconditioner(s.problem, case, case["precond_eps"])
+        s.M.factorize(PREC[case["precision"]])
+        p = torch.from_numpy(s.problem.bodies.reshape(-1, 3)).cuda()
+        s.b = Vec(_dense(case["kernel"], p, x))
+    torch.cuda.synchronize()
+    return s
+
+
+# ---------------------------------------------------------------- one pass
+
+def _solve_m(s, M):
+    """y <- M^-1 x for all columns."""
+    c = s.case
+    s.y.copy(s.x)
+    N.check_gpu(N.gpu().mxg_ulv_solve(N.h2().mxc_solver_ulv(M.handle), s.y.ptr, c["nrhs"], c["n"]))
+
+
+def _apply(s, A):
+    """y <- A x for all columns."""
+    c = s.case
+    N.check_gpu(N.gpu().mxg_h2_matvec(N.h2().mxc_solver_device(A.handle), s.x.ptr, s.y.ptr, c["nrhs"], c["n"],
+                                      PREC[c["precision"]]))
+
+
+def _result(s):
+    return s.y.t if s.case["precision"] == "fp64" else s.y.t.float()
+
+
+def run(s):
+    c, kind = s.case, s.case["kind"]
+    if kind == "matvec":
+        _apply(s, s.A)
+    elif kind == "substitution":
+        _solve_m(s, s.M)
+    elif kind == "factorize":
+        info = s.M.factorize(PREC[c["precision"]])
+        _solve_m(s, s.M)
+        return _result(s), info
+    elif kind == "operator":
+        A = _operator(s.problem, c, c["eps"])
+        _apply(s, A)
+        A.close()
+    elif kind == "preconditioner":
+        M = _preconditioner(s.problem, c, c["eps"])
+        info = M.factorize(PREC[c["precision"]])
+        _solve_m(s, M)
+        M.close()
+        return _result(s), info
+    elif kind == "dense":
+        s.problem.dense_matvec(c["kernel"], DIAG, ALPHA, s.x, s.y)
+    else:
+        s.y.zero()
+        if c["mode"] == "reference":
+            s.A.gmres(s.M, s.b, s.y, 1e-10, 10, 50, N.GMRES_REFERENCE)
+        else:
+            inner = N.MXG_FP32 if s.inner is not None else N.MXG_FP64
+            s.A.gmres_batch(s.M, s.b, s.y, 1e-10, 30, 20, N.GMRES_CGS2, inner, s.inner)
+        return s.y.t  # solved to 1e-10 on the FP64 operator whatever the factors are
+    return _result(s)
+
+
+# ---------------------------------------------------------------- reference values and work
+
+def exact(case, seed):
+    """The dense product for products with the operator and the dense check, the known solution for solves. The
+    preconditioner is an approximation with no value of its own in 64 bits."""
+    kind = case["kind"]
+    if kind in ("substitution", "factorize", "preconditioner"):
+        return None
+    x = _vectors(case, seed)
+    if kind == "gmres":
+        return x
+    p = torch.from_numpy(_tree_order(_points(case, seed), case["leaf"])).cuda()
+    return _dense(case["kernel"], p, x)
+
+
+def _near(case):
+    """Per level, leaves last: the box sizes (above the leaves twice the rank) and the near pairs."""
+    L = tree_levels(case["n"], case["leaf"])
+    tree = build_tree(_points(case, 0).reshape(-1), L)
+    rp, col = csr(False, THETA, L, *tree[1:])
+    body = tree[2].reshape(-1, 2)
+    out = []
+    for l in range(L + 1):
+        a, b = (1 << l) - 1, (2 << l) - 1
+        dims = body[a:b, 1] - body[a:b, 0]
+        if l < L:
+            dims = np.minimum(dims, 2 * case.get("rank", 64))
+        row = np.repeat(np.arange(b - a), np.diff(rp[a:b + 1]))
+        out.append((dims.astype(float), row, col[rp[a]:rp[b]] - a))
+    return out
+
+
+def work(case):
+    """Bytes and operations of one pass: stored blocks read or written once (near blocks and bases; the ranks of an
+    operator's couplings are known only once it is built), vectors in and out, two operations per entry and vector."""
+    n, nrhs, kind = case["n"], case["nrhs"], case["kind"]
+    vec = 16.0 * n * nrhs
+    if kind == "dense":
+        return {"bytes": 24.0 * n + vec, "flops": n * float(n) * (2 * nrhs + 9)}
+    size = {"fp64": 8.0, "fp32": 4.0, "bf16": 2.0}[case["precision"]]
+    levels = _near(case)
+    dims, i, j = levels[-1]
+    near = float((dims[i] * dims[j]).sum())
+    if kind == "matvec":
+        return {"bytes": near * size + vec, "flops": 2.0 * near * nrhs}
+    if kind == "operator":
+        seen = np.bincount(i, weights=dims[j], minlength=len(dims))
+        far = np.minimum(n - seen, 8.0 * case["sampling"])
+        return {"bytes": near * 8.0 + vec, "flops": float((2.0 * dims * dims * far).sum()) + 10.0 * near}
+    if kind == "gmres":
+        size = 4.0 if case["mode"] == "cgs2" and case["precision"] != "fp64" else 8.0
+        return {"bytes": 20.0 * near * size + vec, "flops": 40.0 * near * nrhs}
+    # preconditioner: ranks at their cap. A factorization rotates every near block (all of the diagonal ones, the
+    # skeleton rows and columns of the others) and inverts the rest of each diagonal block; a substitution reads
+    # V, U and the skeleton rows and columns of the off-diagonal blocks.
+    flops = bytes_ = entries = 0.0
+    for l, (M, i, j) in enumerate(levels):
+        s = np.minimum(M, case["rank"] if l else 0)
+        r, off = M - s, i != j
+        bytes_ += float((M[i] * M[j]).sum())
+        entries += float((2 * M * M).sum() + (s[i] * r[j] + r[i] * s[j])[off].sum())
+        flops += float((6 * M * M * M + 2 * r * r * r).sum())
+        flops += float((2 * (s[i] * M[i] * M[j] + s[i] * M[j] * M[j] + M[i] * M[j] * s[j] + r[i] * M[i] * s[j]))[off].sum())
+        flops += float((2 * s[i] * (r[i] * s[j] + r[j] * s[j] + r[j] * r[j] + r[j] * s[i]))[off].sum())
+    if kind == "substitution":
+        return {"bytes": entries * size + vec, "flops": 2.0 * entries * nrhs}
+    fact = 8.0 if case["precision"] == "fp64" else 4.0
+    return {"bytes": 8.0 * bytes_ + fact * bytes_ + size * entries + vec, "flops": flops}
