@@ -86,13 +86,14 @@ struct CpqrTask {
 };
 void cpqr_batched(const std::vector<CpqrTask>& tasks, hipStream_t s);
 
-// LU with partial pivoting and explicit inverse of an n x n block:
-// inv = A^{-1} (ld n); info = 1 when log|det| <= log(DBL_MIN).
+// ---- inverses (lu.hip) ----
+// inv = A^{-1} (n x n, ld n, n <= 1024) with partial pivoting, in FP64
+// arithmetic for either T; info = 1 when log|det| <= log(DBL_MIN).
 template <class T>
 struct LuTask {
-  const T* A;  // input block, ld lda (not modified)
-  T* inv;      // output n x n, ld n
-  T* work;     // n*n + 2n scratch
+  const T* A;    // input block, ld lda (not modified)
+  T* inv;        // output n x n, ld n
+  double* work;  // n * n scratch
   int* info;
   int n, lda;
 };

@@ -7,7 +7,7 @@
 // its batched formulation device_factorize.cu:56-142), for boxes i with
 // M = dims, s = rank, r = M - s, and near pairs (i, j):
 //   1  A_ii <- U_i^T A_ii U_i                          (two batched GEMMs)
-//   2  rr_i^{-1} = (A_ii[s:, s:])^{-1}                 (batched LU + inverse)
+//   2  rr_i^{-1} = (A_ii[s:, s:])^{-1}                 (batched inverse, FP64 arithmetic)
 //   3  V_i = [U_i[:, :s]^T ; rr_i^{-1} U_i[:, s:]^T]   (stored for the solves)
 //   4  A_ii[s:, :s] <- rr^{-1} A_ii[s:, :s];  A_ii[:s, :s] -= A_ii[:s, s:] A_ii[s:, :s]
 //   5  A_ij <- V_i A_ij U_j for j != i, only the ss, sr and rs blocks (the rr
@@ -84,9 +84,10 @@ struct LevelPlan {
   std::vector<GemmList<T>> offa, offb;    // 5, per chunk of pairs
   GemmList<T> sch1, sch2;                 // 6
   Arena* arena = nullptr;  // the scratch: valid until the arena is rewound
-  T* alloc(size_t n) {
+  template <class E = T>
+  E* alloc(size_t n) {
     MXG_REQUIRE(arena, "level plan without scratch arena");
-    return static_cast<T*>(arena->take(std::max<size_t>(n, 1) * sizeof(T)));
+    return static_cast<E*>(arena->take(std::max<size_t>(n, 1) * sizeof(E)));
   }
   void merge(LevelPlan&& o) {
     rot1.append(o.rot1);
@@ -371,15 +372,15 @@ struct UlvImpl : UlvBase {
       size_t wsz = 0;
       for (long long i = 0; i < nb; i++) {
         const long long r = M_(i) - S_(i);
-        wsz += (size_t)r * r + 2 * r;
+        wsz += (size_t)r * r;
       }
-      T* work = P.alloc(wsz);
+      double* work = P.template alloc<double>(wsz);
       size_t wo = 0;
       for (long long i = 0; i < nb; i++) {
         const int M = M_(i), sI = S_(i), r = M - sI;
         if (r == 0) continue;
         P.lu.push_back(LuTask<T>{Aij(H.diag[i]) + sI + (long long)sI * M, RRi(i), work + wo, F.info.p + i, r, M});
-        wo += (size_t)r * r + 2 * r;
+        wo += (size_t)r * r;
       }
     }
     // 3: V = [U[:, :s]^T ; rr^{-1} U[:, s:]^T]
