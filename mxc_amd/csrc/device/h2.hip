@@ -66,57 +66,50 @@ __global__ void k_leaf_init(int nb, const long long* __restrict__ offX, const lo
 
 // Interpolative decomposition post-processing of one box (h2matrix.cpp:92-116).
 struct PostTask {
-  const double* R0;  // CPQR output, K x M (ld ldr)
   const int* perm;   // M
   double* Q;         // M x M (holds Q_in on entry)
   double* R;         // M x M
   int* S;            // M skeleton indices
   int* Stmp;         // M scratch
-  double* T;         // r x (M - r) scratch
-  double* W;         // M x r: P [I; T^T]
-  int M, r, ldr, mode;  // mode 1: rank 0 or M; mode 2: 0 < r < M interpolative; mode 3: same, orthogonal
+  const double* T;   // R11^{-1} R12, r x (M - r)
+  double* W;         // mode 3, M x r: P [I; T^T]
+  int M, r, mode;    // mode 1: rank 0 or M; mode 2: 0 < r < M interpolative; mode 3: same, orthogonal
+  int pad;
 };
 
+// The entries of a box are independent of each other: POST_BLOCKS workgroups
+// share them; the first also permutes the skeleton indices.
+constexpr int POST_BLOCKS = 8;
 __global__ void __launch_bounds__(256) k_post(const PostTask* __restrict__ tasks) {
   const PostTask t = tasks[blockIdx.x];
   const int M = t.M, r = t.r;
+  const int first = blockIdx.y * 256 + threadIdx.x, step = gridDim.y * 256;
   if (t.mode == 1) {
     // R = triu(Q_in), Q = I
-    for (long long e = threadIdx.x; e < (long long)M * M; e += 256) {
-      const int i = (int)(e % M), j = (int)(e / M);
+    for (int e = first; e < M * M; e += step) {
+      const int i = e % M, j = e / M;
       t.R[e] = (i <= j) ? t.Q[e] : 0.;
+      t.Q[e] = (i == j) ? 1. : 0.;
     }
-    __syncthreads();
-    for (long long e = threadIdx.x; e < (long long)M * M; e += 256) t.Q[e] = ((e % M) == (e / M)) ? 1. : 0.;
     return;
   }
-  // T = R11^{-1} R12, one column per thread (back substitution)
-  for (int c = threadIdx.x; c < M - r; c += 256) {
-    double* x = t.T + (long long)c * r;
-    const double* b = t.R0 + (long long)(r + c) * t.ldr;
-    for (int i = r - 1; i >= 0; i--) {
-      double s = b[i];
-      for (int j = i + 1; j < r; j++) s -= t.R0[i + (long long)j * t.ldr] * x[j];
-      x[i] = s / t.R0[i + (long long)i * t.ldr];
-    }
-  }
-  for (int j = threadIdx.x; j < M; j += 256) t.Stmp[j] = t.S[t.perm[j]];
-  __syncthreads();
-  for (int j = threadIdx.x; j < M; j += 256) t.S[j] = t.Stmp[j];
-  // W = P [I; T^T]: row perm[j] of W is row j of [I; T^T]
-  for (long long e = threadIdx.x; e < (long long)M * r; e += 256) {
-    const int j = (int)(e % M), c = (int)(e / M);
-    const double v = (j < r) ? (j == c ? 1. : 0.) : t.T[c + (long long)(j - r) * r];
-    t.W[t.perm[j] + (long long)c * M] = v;
-  }
-  if (t.mode == 2) {
+  if (blockIdx.y == 0) {
+    for (int j = threadIdx.x; j < M; j += 256) t.Stmp[j] = t.S[t.perm[j]];
     __syncthreads();
-    for (long long e = threadIdx.x; e < (long long)M * M; e += 256) {
-      const int i = (int)(e % M), j = (int)(e / M);
-      t.Q[e] = (j < r) ? t.W[i + (long long)j * M] : 0.;
+    for (int j = threadIdx.x; j < M; j += 256) t.S[j] = t.Stmp[j];
+  }
+  // P [I; T^T]: row perm[j] is row j of [I; T^T]; mode 2 writes it into Q
+  double* W = t.mode == 2 ? t.Q : t.W;
+  for (int e = first; e < M * r; e += step) {
+    const int j = e % M, c = e / M;
+    W[t.perm[j] + (long long)c * M] = (j < r) ? (j == c ? 1. : 0.) : t.T[c + (long long)(j - r) * r];
+  }
+  if (t.mode == 2)
+    for (int e = first; e < M * M; e += step) {
+      const int i = e % M, j = e / M;
+      if (j >= r) t.Q[e] = 0.;
       t.R[e] = (i == j && j < r) ? 1. : 0.;
     }
-  }
 }
 
 // QT_i = Q_i[:, :k]^T (k x M, column major), the row-major basis the upward
@@ -405,6 +398,7 @@ void construct_basis(mxg_h2_s* h, Level& Lv, long long l, const FarRows& fr, dou
 
     // post-processing (h2matrix.cpp:92-116)
     std::vector<PostTask> posts;
+    std::vector<TrTask> solves;
     std::vector<long long> orth_boxes;
     size_t tneed = 0, wneed = 0;
     for (long long i = b0; i < b1; i++) {
@@ -419,7 +413,7 @@ void construct_basis(mxg_h2_s* h, Level& Lv, long long l, const FarRows& fr, dou
     }
     DevBuf<double> Tm, Wm, P, ptau;
     Tm.alloc(std::max<size_t>(tneed, 1));
-    Wm.alloc_zero(std::max<size_t>(wneed, 1), s);
+    Wm.alloc(std::max<size_t>(orth ? wneed : 0, 1));
     std::vector<size_t> wof(nb, 0);
     size_t to = 0, wo = 0;
     for (long long i = b0; i < b1; i++) {
@@ -432,13 +426,12 @@ void construct_basis(mxg_h2_s* h, Level& Lv, long long l, const FarRows& fr, dou
       pt.M = (int)M;
       pt.r = (int)r;
       if (0 < r && r < M) {
-        pt.R0 = G.p + goff[i - b0];
-        pt.ldr = (int)ldg[i];
+        solves.push_back(TrTask{G.p + goff[i - b0], Tm.p + to, (int)r, (int)(M - r), (int)ldg[i], 0});
         pt.perm = d_perm.p + Lv.offX[i];
         pt.S = Lv.S.p + Lv.offX[i];
         pt.Stmp = d_stmp.p + Lv.offX[i];
         pt.T = Tm.p + to;
-        pt.W = Wm.p + wo;
+        pt.W = orth ? Wm.p + wo : nullptr;
         pt.mode = orth ? 3 : 2;
         wof[i] = wo;
         to += (size_t)r * (M - r);
@@ -449,10 +442,11 @@ void construct_basis(mxg_h2_s* h, Level& Lv, long long l, const FarRows& fr, dou
       }
       posts.push_back(pt);
     }
+    trsolve_batched(solves, s);
     if (!posts.empty()) {
       DevBuf<PostTask> dt;
       dt.upload(posts, s);
-      hipLaunchKernelGGL(k_post, dim3((unsigned)posts.size()), dim3(256), 0, s, dt.p);
+      hipLaunchKernelGGL(k_post, dim3((unsigned)posts.size(), POST_BLOCKS), dim3(256), 0, s, dt.p);
       MXG_HIP(hipGetLastError());
       MXG_HIP(hipStreamSynchronize(s));
     }

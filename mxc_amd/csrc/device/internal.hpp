@@ -47,7 +47,7 @@ template <class T>
 void gemm_batched(const std::vector<GemmTask<T>>& tasks, const std::vector<GemmSeg<T>>& segs, hipStream_t s,
                   bool bf16 = false, Stage* st = nullptr);
 
-// ---- dense factorizations, one workgroup per matrix (lapack.hip) ----
+// ---- Householder factorizations (qr.hip) ----
 // Householder QR of an m x n column-major matrix in place (R on/above the
 // diagonal, reflectors below), Eigen's reflector convention.
 struct QrTask {
@@ -85,6 +85,16 @@ struct CpqrTask {
   int pad;
 };
 void cpqr_batched(const std::vector<CpqrTask>& tasks, hipStream_t s);
+
+// X = R11^{-1} R12 (r x n, ld r) of a pivoted QR: R11 = triu(R0[:r, :r]),
+// R12 = R0[:r, r : r + n].
+struct TrTask {
+  const double* R0;
+  double* X;
+  int r, n, ldr;
+  int pad;
+};
+void trsolve_batched(const std::vector<TrTask>& tasks, hipStream_t s);
 
 // ---- inverses (lu.hip) ----
 // inv = A^{-1} (n x n, ld n, n <= 1024) with partial pivoting, in FP64
