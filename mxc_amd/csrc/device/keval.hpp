@@ -1,0 +1,61 @@
+// Kernel entries for the kernels that evaluate them by the billion: the value
+// of kernel_eval to an ulp or two, without its correctly rounded square root and
+// division and the general exponential's range checks (about 35 vector
+// instructions an entry for Yukawa, 70 with kernel_eval).
+#pragma once
+
+#include "common.hpp"
+
+namespace mxg {
+
+// 2^f for |f| <= 1/2: interpolation at 12 Chebyshev nodes (error 2e-17)
+__device__ inline double exp2_poly(double f) {
+  double p = 4.4558179083360645e-10;
+  p = fma(p, f, 7.074194297288521e-09);
+  p = fma(p, f, 1.0178057087733941e-07);
+  p = fma(p, f, 1.3215432535912375e-06);
+  p = fma(p, f, 1.5252733841556773e-05);
+  p = fma(p, f, 0.00015403530463724353);
+  p = fma(p, f, 0.001333355814640647);
+  p = fma(p, f, 0.009618129107587256);
+  p = fma(p, f, 0.055504108664821625);
+  p = fma(p, f, 0.24022650695910158);
+  p = fma(p, f, 0.6931471805599453);
+  return fma(p, f, 1.0);
+}
+
+// What the evaluation needs of a kernel: K(0), and -alpha log2(e) as the
+// unevaluated sum of two doubles.
+struct EvalArgs {
+  double diag, ch, cl;
+};
+
+inline EvalArgs eval_args(mxg_kernel_t k) {
+  // the product's rounding error and log2(e)'s own tail make the second part
+  const double L2E = 1.4426950408889634, L2E_TAIL = 2.0355273740931033e-17, ch = -k.alpha * L2E;
+  return EvalArgs{k.id == MXG_KERNEL_GAUSSIAN ? 1.0001 : k.diag, ch, std::fma(-k.alpha, L2E, -ch) - k.alpha * L2E_TAIL};
+}
+
+// 1 / sqrt(x) from the hardware's estimate and one step of third order.
+__device__ inline double rsqrt_refined(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+// K(d) 2^shift from the squared distance (not zero).
+template <int KID>
+__device__ inline double kernel_scaled(double d2, const EvalArgs& k, int shift) {
+  if constexpr (KID == MXG_KERNEL_LAPLACE) {
+    return ldexp(rsqrt_refined(d2), shift);
+  } else {
+    const double v = KID == MXG_KERNEL_YUKAWA ? rsqrt_refined(d2) : 1.0;
+    const double d = KID == MXG_KERNEL_YUKAWA ? d2 * v : d2;
+    const double y = d * k.ch, r = rint(y);
+    double p = exp2_poly(fma(d, k.cl, fma(d, k.ch, -r)));
+    if constexpr (KID == MXG_KERNEL_YUKAWA) p *= v;
+    return ldexp(p, (int)r + shift);
+  }
+}
+
+}  // namespace mxg

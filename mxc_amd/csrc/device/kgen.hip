@@ -7,6 +7,7 @@
 #include <mutex>
 
 #include "internal.hpp"
+#include "keval.hpp"
 
 namespace mxg {
 namespace {
@@ -39,48 +40,82 @@ __global__ void __launch_bounds__(256) k_gen(const GenTask* __restrict__ tasks, 
 // Dense check: partial sums of Y = K X over column chunks, then a
 // fixed-order reduction (deterministic; no atomics). Each kernel entry is
 // evaluated once and applied to the NR right-hand sides of the launch.
+//
+// The sums run on the FP64 matrix cores, beside the vector units that evaluate
+// the entries: lane l evaluates the entry of row l mod 16 and column l / 16 of
+// a 16 x 4 block, which is the A operand of v_mfma_f64_16x16x4f64 as it
+// stands; the right-hand sides are the 16 columns of B (zero past NR). A wave
+// holds 64 rows, so that a column's coordinates and right-hand sides are read
+// from LDS once for four blocks. Bound by the evaluation (36 vector
+// instructions an entry; without the register limit below the accumulators move
+// through the accumulation registers, 16 more): N = 65536 Yukawa, 8 right-hand
+// sides, 6.2 ms, where evaluation with kernel_eval and sums on the vector units
+// took 11.0.
 constexpr int DM_ROWS = 256, DM_CHUNK = 8192;
+typedef double d4_t __attribute__((ext_vector_type(4)));
 
 // Rows row0 + blockIdx.x * DM_ROWS + t of the launch; partial sums of chunk c
 // and right-hand side q at part[(c * NR + q) * ldp + (row - row0)].
-template <int NR>
-__global__ void __launch_bounds__(256) k_dense_partial(const double* __restrict__ bodies, const double* __restrict__ x,
-                                                       long long ldx, long long n, int kid, double diag, double alpha,
-                                                       long long row0, long long rows, long long ldp,
-                                                       double* __restrict__ part) {
+template <int KID, int NR>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_dense_partial(const double* __restrict__ bodies, const double* __restrict__ x,
+                                                       long long ldx, long long n, EvalArgs ke, long long row0,
+                                                       long long rows, long long ldp, double* __restrict__ part) {
   __shared__ double sp[256 * 3];
-  __shared__ double sx[NR][256];
-  const long long li = (long long)blockIdx.x * DM_ROWS + threadIdx.x;
-  const long long i = row0 + li;
-  const bool live = li < rows && i < n;
-  long long j0 = (long long)blockIdx.y * DM_CHUNK;
-  long long j1 = min(j0 + DM_CHUNK, n);
-  double p[3] = {0., 0., 0.};
-  if (live) { p[0] = bodies[3 * i]; p[1] = bodies[3 * i + 1]; p[2] = bodies[3 * i + 2]; }
-  double acc[NR];
+  __shared__ double sx[256 * NR];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 15, lk = lane >> 4;
+  const long long base = (long long)blockIdx.x * DM_ROWS + wave * 64;
+  const long long j0 = (long long)blockIdx.y * DM_CHUNK, j1 = min(j0 + DM_CHUNK, n);
+  double p[4][3];
+  d4_t acc[4];
 #pragma unroll
-  for (int q = 0; q < NR; q++) acc[q] = 0.;
+  for (int r = 0; r < 4; r++) {
+    const long long i = min(row0 + base + 16 * r + lr, n - 1);
+#pragma unroll
+    for (int d = 0; d < 3; d++) p[r][d] = bodies[3 * i + d];
+    acc[r] = d4_t{0., 0., 0., 0.};
+  }
   for (long long jt = j0; jt < j1; jt += 256) {
-    int cnt = (int)min((long long)256, j1 - jt);
+    const int cnt = (int)min((long long)256, j1 - jt);
     __syncthreads();
-    if ((int)threadIdx.x < cnt) {
-      long long j = jt + threadIdx.x;
-      sp[3 * threadIdx.x] = bodies[3 * j];
-      sp[3 * threadIdx.x + 1] = bodies[3 * j + 1];
-      sp[3 * threadIdx.x + 2] = bodies[3 * j + 2];
+    {  // columns past the chunk repeat its last one, with zero right-hand sides
+      const long long j = min(jt + tid, j1 - 1);
 #pragma unroll
-      for (int q = 0; q < NR; q++) sx[q][threadIdx.x] = x[j + q * ldx];
+      for (int d = 0; d < 3; d++) sp[3 * tid + d] = bodies[3 * j + d];
+#pragma unroll
+      for (int q = 0; q < NR; q++) sx[tid * NR + q] = tid < cnt ? x[j + q * ldx] : 0.;
     }
     __syncthreads();
-    for (int c = 0; c < cnt; c++) {
-      const double kv = kernel_eval(kid, diag, alpha, dist2(p, &sp[3 * c]));
+    for (int c = 0; c < cnt; c += 4) {
+      const double* s = sp + 3 * (c + lk);
+      const double xb = lr < NR ? sx[(c + lk) * NR + (lr < NR ? lr : 0)] : 0.;
+      double d2[4], v[4];
 #pragma unroll
-      for (int q = 0; q < NR; q++) acc[q] += kv * sx[q][c];
+      for (int r = 0; r < 4; r++) {
+        const double dx = p[r][0] - s[0], dy = p[r][1] - s[1], dz = p[r][2] - s[2];
+        d2[r] = dx * dx + dy * dy + dz * dz;
+        v[r] = kernel_scaled<KID>(d2[r], ke, 0);
+      }
+      if (__any(d2[0] == 0. || d2[1] == 0. || d2[2] == 0. || d2[3] == 0.)) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) v[r] = d2[r] == 0. ? ke.diag : v[r];
+      }
+      if (c + 4 > cnt) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) v[r] = c + lk < cnt ? v[r] : 0.;
+      }
+#pragma unroll
+      for (int r = 0; r < 4; r++) acc[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(v[r], xb, acc[r], 0, 0, 0);
     }
   }
-  if (live)
+  // entry q of lane l: row l / 16 + 4 q of the block, right-hand side l mod 16
+  if (lr < NR)
 #pragma unroll
-    for (int q = 0; q < NR; q++) part[((long long)blockIdx.y * NR + q) * ldp + li] = acc[q];
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const long long li = base + 16 * r + lk + 4 * q;
+        if (li < rows && row0 + li < n) part[((long long)blockIdx.y * NR + lr) * ldp + li] = acc[r][q];
+      }
 }
 
 // y[row0 + li] = sum over the chunks, in order, of the partial sums of the row
@@ -103,12 +138,25 @@ void dense_group(mxg_ctx_t ctx, mxg_kernel_t k, const double* d_bodies, long lon
                  double* y, long long ldy, int nr, long long row0, long long rows, double* part, long long ldp) {
   const int nchunks = (int)ceil_div(n, DM_CHUNK);
   const dim3 g(ceil_div(rows, DM_ROWS), nchunks), b(256);
-  switch (nr) {
-    case 8: hipLaunchKernelGGL(k_dense_partial<8>, g, b, 0, ctx->stream, d_bodies, x, ldx, n, k.id, k.diag, k.alpha, row0, rows, ldp, part); break;
-    case 4: hipLaunchKernelGGL(k_dense_partial<4>, g, b, 0, ctx->stream, d_bodies, x, ldx, n, k.id, k.diag, k.alpha, row0, rows, ldp, part); break;
-    case 2: hipLaunchKernelGGL(k_dense_partial<2>, g, b, 0, ctx->stream, d_bodies, x, ldx, n, k.id, k.diag, k.alpha, row0, rows, ldp, part); break;
-    default: hipLaunchKernelGGL(k_dense_partial<1>, g, b, 0, ctx->stream, d_bodies, x, ldx, n, k.id, k.diag, k.alpha, row0, rows, ldp, part); break;
+  const EvalArgs ke = eval_args(k);
+#define MXG_DENSE(ID, NN) \
+  hipLaunchKernelGGL((k_dense_partial<ID, NN>), g, b, 0, ctx->stream, d_bodies, x, ldx, n, ke, row0, rows, ldp, part)
+#define MXG_DENSE_ID(ID)              \
+  switch (nr) {                       \
+    case 8: MXG_DENSE(ID, 8); break;  \
+    case 4: MXG_DENSE(ID, 4); break;  \
+    case 2: MXG_DENSE(ID, 2); break;  \
+    default: MXG_DENSE(ID, 1); break; \
   }
+  if (k.id == MXG_KERNEL_GAUSSIAN) {
+    MXG_DENSE_ID(MXG_KERNEL_GAUSSIAN)
+  } else if (k.id == MXG_KERNEL_YUKAWA) {
+    MXG_DENSE_ID(MXG_KERNEL_YUKAWA)
+  } else {
+    MXG_DENSE_ID(MXG_KERNEL_LAPLACE)
+  }
+#undef MXG_DENSE_ID
+#undef MXG_DENSE
   MXG_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_dense_reduce, dim3(ceil_div(rows, 256)), dim3(256), 0, ctx->stream, part, row0, rows, ldp, nchunks, nr,
                      y, ldy);

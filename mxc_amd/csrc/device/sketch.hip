@@ -49,6 +49,7 @@
 #include <map>
 
 #include "internal.hpp"
+#include "keval.hpp"
 #include "wave.hpp"
 
 namespace mxg {
@@ -91,50 +92,6 @@ __global__ void __launch_bounds__(256) k_sketch_signs(u4* __restrict__ signs, in
 // the word are the integer's signed base-256 digits.
 constexpr unsigned DIGITS = 0x80808080u;
 constexpr double MAGIC = 6755399441055744.0 + 2155905152.0;  // 1.5 2^52 + DIGITS
-
-// 2^f for |f| <= 1/2: interpolation at 12 Chebyshev nodes (error 2e-17)
-__device__ inline double exp2_poly(double f) {
-  double p = 4.4558179083360645e-10;
-  p = fma(p, f, 7.074194297288521e-09);
-  p = fma(p, f, 1.0178057087733941e-07);
-  p = fma(p, f, 1.3215432535912375e-06);
-  p = fma(p, f, 1.5252733841556773e-05);
-  p = fma(p, f, 0.00015403530463724353);
-  p = fma(p, f, 0.001333355814640647);
-  p = fma(p, f, 0.009618129107587256);
-  p = fma(p, f, 0.055504108664821625);
-  p = fma(p, f, 0.24022650695910158);
-  p = fma(p, f, 0.6931471805599453);
-  return fma(p, f, 1.0);
-}
-
-// What the evaluation needs of a kernel: K(0), and -alpha log2(e) as the
-// unevaluated sum of two doubles.
-struct EvalArgs {
-  double diag, ch, cl;
-};
-
-// 1 / sqrt(x) from the hardware's estimate and one step of third order.
-__device__ inline double rsqrt_refined(double x) {
-  const double y = __builtin_amdgcn_rsq(x);
-  const double e = fma(-x * y, y, 1.0);
-  return fma(y * e, fma(e, 0.375, 0.5), y);
-}
-
-// K(d) 2^shift from the squared distance (not zero).
-template <int KID>
-__device__ inline double kernel_scaled(double d2, const EvalArgs& k, int shift) {
-  if constexpr (KID == MXG_KERNEL_LAPLACE) {
-    return ldexp(rsqrt_refined(d2), shift);
-  } else {
-    const double v = KID == MXG_KERNEL_YUKAWA ? rsqrt_refined(d2) : 1.0;
-    const double d = KID == MXG_KERNEL_YUKAWA ? d2 * v : d2;
-    const double y = d * k.ch, r = rint(y);
-    double p = exp2_poly(fma(d, k.cl, fma(d, k.ch, -r)));
-    if constexpr (KID == MXG_KERNEL_YUKAWA) p *= v;
-    return ldexp(p, (int)r + shift);
-  }
-}
 
 // 4 x 4 bytes transposed: out[s] = byte s of a, b, c, d.
 __device__ inline void bytes_of(unsigned a, unsigned b, unsigned c, unsigned d, unsigned (&out)[4]) {
@@ -292,7 +249,7 @@ __global__ void __launch_bounds__(512) k_sketch(const SketchTask* __restrict__ t
       for (int e = 0; e < E; e++) {
         const int tt = 16 * tg + sub * E + e;
         if (Xr[b][tt][0] == x0 && Xr[b][tt][1] == x1 && Xr[b][tt][2] == x2)
-          v[e] = ldexp(KID == MXG_KERNEL_GAUSSIAN ? 1.0001 : ke.diag, shift - 30);
+          v[e] = ldexp(ke.diag, shift - 30);
       }
     }
     if (tb + KT > tk.t1) {
@@ -430,9 +387,7 @@ template <int KID>
 void launch_sketch(int shape, unsigned grid, const SketchTask* tasks, const double* bodies, mxg_kernel_t k,
                    const u4* signs, int nu, hipStream_t s) {
   const dim3 g(grid), blk(512);
-  // -alpha log2(e) = ch + cl: the product's rounding error and log2(e)'s own tail
-  const double L2E = 1.4426950408889634, L2E_TAIL = 2.0355273740931033e-17, ch = -k.alpha * L2E;
-  const EvalArgs ke{k.diag, ch, std::fma(-k.alpha, L2E, -ch) - k.alpha * L2E_TAIL};
+  const EvalArgs ke = eval_args(k);
   switch (shape) {
     case 0: hipLaunchKernelGGL((k_sketch<KID, 4, 1, 2, 64>), g, blk, 0, s, tasks, bodies, k.alpha, ke, signs, nu); break;
     case 1: hipLaunchKernelGGL((k_sketch<KID, 8, 1, 4, 64>), g, blk, 0, s, tasks, bodies, k.alpha, ke, signs, nu); break;
