@@ -89,13 +89,26 @@ constexpr int unroll() {
 __device__ inline int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 
 // Stage columns [cb, cb + cn) of the NR right-hand sides as vs[c NR + k], so
-// that a column's NR values are one broadcast LDS read.
+// that a column's NR values are one broadcast LDS read. A thread takes whole
+// columns, so that its NR loads are in flight together.
+template <class T, int NR, class VF>
+__device__ inline void stage_cols(T* vs, int first, int step, int cn, VF vfun) {
+  typedef typename Vec<T, NR>::type WT;
+  for (int c = first; c < cn; c += step) {
+    WT w;
+    if constexpr (NR == 1) {
+      w = vfun(c, 0);
+    } else {
+#pragma unroll
+      for (int k = 0; k < NR; k++) w[k] = vfun(c, k);
+    }
+    *reinterpret_cast<WT*>(vs + c * NR) = w;
+  }
+}
 template <class T, int NR, class VF>
 __device__ inline void stage_v(T* vs, int cb, int cn, VF vfun) {
   __syncthreads();
-#pragma unroll
-  for (int k = 0; k < NR; k++)
-    for (int c = threadIdx.x; c < cn; c += 256) vs[c * NR + k] = vfun(cb + c, k);
+  stage_cols<T, NR>(vs, threadIdx.x, 256, cn, [&](int c, int k) { return vfun(cb + c, k); });
   __syncthreads();
 }
 
@@ -304,9 +317,7 @@ __device__ inline void wave_gemv(const PairJob& t, int c0, T* __restrict__ vw) {
   for (int cb = 0; cb < m; cb += CW) {
     const int cn = min(CW, m - cb);
     wave_lds_sync();
-#pragma unroll
-    for (int k = 0; k < NR; k++)
-      for (int c = lane; c < cn; c += 64) vw[c * NR + k] = vb[cb + c + (long long)k * t.ldv];
+    stage_cols<T, NR>(vw, lane, 64, cn, [&](int c, int k) { return vb[cb + c + (long long)k * t.ldv]; });
     wave_lds_sync();
     // lanes past the column's end load its first V rows; their sums are dropped
     const S* Bc = B + (long long)cb * t.ld + (active ? r : 0);
@@ -339,7 +350,8 @@ __device__ inline void wave_gemv(const PairJob& t, int c0, T* __restrict__ vw) {
         o[0] = acc[k];
       } else {
 #pragma unroll
-        for (int e = 0; e < V; e++) o[e] = acc[k][e];
+        for (int e = 0; e < V; e++)
+          if (r + e < n) o[e] = acc[k][e];
       }
     }
 }
@@ -599,6 +611,141 @@ __device__ inline T sum_terms(const T* __restrict__ t, const long long* __restri
   return (a0 + a1) + (a2 + a3);
 }
 
+// The same sum with the offsets of the box's terms in LDS (n of them): the loads
+// of the terms then wait for no load of an offset.
+template <class T>
+__device__ inline T sum_terms_lds(const T* __restrict__ t, const long long* toff, int n, long long off) {
+  T a0 = T(0), a1 = T(0), a2 = T(0), a3 = T(0);
+  int p = 0;
+#pragma unroll 2
+  for (; p + 3 < n; p += 4) {
+    a0 += t[toff[p] + off];
+    a1 += t[toff[p + 1] + off];
+    a2 += t[toff[p + 2] + off];
+    a3 += t[toff[p + 3] + off];
+  }
+  for (; p < n; p++) a0 += t[toff[p] + off];
+  return (a0 + a1) + (a2 + a3);
+}
+
+constexpr int TOFFS = 512;  // term offsets staged in LDS; longer lists are read from memory
+__device__ inline bool stage_toff(long long* lds, const long long* __restrict__ toff, long long p0, long long p1) {
+  if (p1 - p0 > TOFFS) return false;
+  for (int p = threadIdx.x; p < (int)(p1 - p0); p += 256) lds[p] = toff[p0 + p];
+  return true;
+}
+
+// ---- levels of few boxes ----
+// A level of up to some hundred boxes leaves most of the GPU idle, and its
+// launches are bound by their chain of dependent memory round trips, not by
+// bytes: with one wave per 32 rows and four columns in flight a lane, a 200 x
+// 200 box takes ten round trips. Here a whole workgroup takes 32 (at most 64)
+// rows, every lane has U columns in flight, and the first of them are requested
+// before the right-hand sides are staged, so that most products wait for memory
+// twice: once for the descriptors, once for the data. (N = 20000, rank 100:
+// the products of a substitution's upper levels 12 -> 5 us each; with 8 right-hand
+// sides 13 -> 7.)
+
+constexpr int LAT_ROWS = 64;  // rows of a job at most
+template <class T>
+constexpr int lat_elems() {
+  return 16384 / (int)sizeof(T);
+}
+// columns a lane has in flight: as many as the registers of NR accumulators leave
+template <class T, int V, int NR>
+constexpr int lat_unroll() {
+  return NR * V * (int)sizeof(T) >= 128 ? 8 : 16;
+}
+
+// out[r, k] = sum_c B[r, c] v(c, k) for r < n <= min(64 V, LAT_ROWS) by the
+// whole workgroup: a column takes lpc lanes, the 4 * 64 / lpc lane groups take
+// every such column in order; the groups' sums are added in a fixed order, which
+// does not depend on NR. stage(cb, cn) puts v(cb + c, k) into xs[c NR + k], with
+// barriers before and after; emit(r, k, sum).
+template <class T, class S, int V, int NR, class SF, class EF>
+__device__ inline void lat_gemv(const S* __restrict__ B, long long ld, int n, int m, T* xs, SF stage, EF emit) {
+  typedef typename Vec<T, V>::type VT;
+  typedef typename Vec<T, NR>::type WT;
+  typedef typename Raw<T, S, V>::type RT;
+  constexpr int U = lat_unroll<T, V, NR>();
+  constexpr int CW = lat_elems<T>() / NR;
+  static_assert(CW % 256 == 0, "column chunks must keep every lane group's column sequence");
+  static_assert(4 * LAT_ROWS * NR <= lat_elems<T>(), "the waves' sums must fit the staged values' place");
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int nv = (n + V - 1) / V;
+  int lpc = 1;
+  while (lpc < nv) lpc <<= 1;
+  const int G = 64 / lpc, NG = 4 * G, gg = wave * G + lane / lpc, r = (lane % lpc) * V;
+  const bool active = r < n;
+  const S* Br = B + (active ? r : 0);
+  auto load = [&](RT (&a)[U], int c0) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int c = c0 + u * NG;
+      a[u] = c < m ? load_raw<T, S, V>(Br + (long long)c * ld) : RT(0);
+    }
+  };
+  VT acc[NR];
+#pragma unroll
+  for (int k = 0; k < NR; k++) acc[k] = VT(0);
+  RT a[U];
+  load(a, gg);
+  for (int cb = 0; cb < m; cb += CW) {
+    const int cn = min(CW, m - cb);
+    stage(cb, cn);
+    for (int c = gg; c < cn; c += U * NG) {
+      if (cb + c != gg) load(a, cb + c);
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        if (c + u * NG < cn) fma_col<T, NR>(acc, cvt<T, S, V>(a[u]), lds_row<T, NR>(xs + (c + u * NG) * NR));
+    }
+  }
+  for (int sh = lpc; sh < 64; sh <<= 1)
+#pragma unroll
+    for (int k = 0; k < NR; k++) {
+      if constexpr (V == 1) {
+        acc[k] += __shfl_xor(acc[k], sh);
+      } else {
+#pragma unroll
+        for (int e = 0; e < V; e++) acc[k][e] += __shfl_xor(acc[k][e], sh);
+      }
+    }
+  __syncthreads();  // the staged values have been read
+  if (lane < lpc && active)
+#pragma unroll
+    for (int k = 0; k < NR; k++) {
+      if constexpr (V == 1) {
+        xs[(wave * NR + k) * LAT_ROWS + r] = acc[k];
+      } else {
+#pragma unroll
+        for (int e = 0; e < V; e++)
+          if (r + e < n) xs[(wave * NR + k) * LAT_ROWS + r + e] = acc[k][e];
+      }
+    }
+  __syncthreads();
+  for (int e = threadIdx.x; e < n * NR; e += 256) {
+    const int rr = e % n, k = e / n;
+    const T* q = xs + k * LAT_ROWS + rr;
+    emit(rr, k, (q[0] + q[NR * LAT_ROWS]) + (q[2 * NR * LAT_ROWS] + q[3 * NR * LAT_ROWS]));
+  }
+}
+
+// Right-hand sides c0 .. c0 + NR - 1 of every job, one workgroup per job (n <= LAT_ROWS).
+template <class T, class S, int NR>
+__global__ void __launch_bounds__(256) k_pair_gemv_lat(const PairJob* __restrict__ jobs, int c0) {
+  __shared__ __align__(16) T xs[lat_elems<T>()];
+  const PairJob t = jobs[blockIdx.x];
+  const S* B = static_cast<const S*>(t.B);
+  const T* vb = static_cast<const T*>(t.v) + (long long)c0 * t.ldv;
+  T* ob = static_cast<T*>(t.out) + (long long)c0 * t.ldo;
+  auto stage = [&](int cb, int cn) { stage_v<T, NR>(xs, cb, cn, [&](int c, int k) { return vb[c + (long long)k * t.ldv]; }); };
+  auto emit = [&](int r, int k, T s) { ob[r + (long long)k * t.ldo] = s; };
+  if (t.vec)
+    lat_gemv<T, S, vwidth<S>(), NR>(B, t.ld, t.n, t.m, xs, stage, emit);
+  else
+    lat_gemv<T, S, 1, NR>(B, t.ld, t.n, t.m, xs, stage, emit);
+}
+
 // Strides (elements) between right-hand sides of the vectors of a per-box sum.
 struct Strides {
   long long a, b, c, d;
@@ -642,46 +789,58 @@ __global__ void __launch_bounds__(256) k_comb_down(const int* __restrict__ dims,
   wg_gemv<T, T, V, NR>(Q + offQ[i], M, M, k, [&](int c, int q) { return w[c + q * kmax]; }, emit, red, vs);
 }
 
-// Forward substitution, skeleton part: z_i = x_i[:s] - sum_near t_p.
-// Strides: a = x, b = t, c = z.
+// Forward substitution, skeleton part: z_i = x_i[:s] - sum_near t_p, 256
+// elements per workgroup. Strides: a = x, b = t, c = z.
 template <class T>
 __global__ void __launch_bounds__(256) k_comb_fwd(const int* __restrict__ ranks, const long long* __restrict__ offX,
                                                   const long long* __restrict__ offZ, const long long* __restrict__ nrp,
                                                   const long long* __restrict__ toff, const T* __restrict__ x,
                                                   const T* __restrict__ t, T* __restrict__ z, Strides ld, int nr) {
+  __shared__ long long to[TOFFS];
   const int i = blockIdx.x;
   const int s = ranks[i];
-  for (int e = threadIdx.x; e < s * nr; e += 256) {
-    const int r = e % s, q = e / s;
-    T acc = x[offX[i] + r + q * ld.a];
-    acc -= sum_terms(t, toff, nrp[i], nrp[i + 1], r + q * ld.b);
-    z[offZ[i] + r + q * ld.c] = acc;
-  }
+  if ((int)blockIdx.y * 256 >= s * nr) return;
+  const long long p0 = nrp[i], p1 = nrp[i + 1];
+  const bool staged = stage_toff(to, toff, p0, p1);
+  __syncthreads();
+  const int e = blockIdx.y * 256 + threadIdx.x;
+  if (e >= s * nr) return;
+  const int r = e % s, q = e / s;
+  const long long off = r + q * ld.b;
+  T acc = x[offX[i] + r + q * ld.a];
+  acc -= staged ? sum_terms_lds(t, to, (int)(p1 - p0), off) : sum_terms(t, toff, p0, p1, off);
+  z[offZ[i] + r + q * ld.c] = acc;
 }
 
 // Backward substitution, the vector only: v_i = [w_i ; x_i[s:] - sum_near t_p]
 // into v (offsets offX), for a separate launch of the products U_i v_i; the
-// same arithmetic as the assembly in k_comb_bwd. Strides: a = x, b = w,
-// c = t, d = v.
+// same arithmetic as the assembly in k_comb_bwd and k_bwd_lat. Strides: a = x, b
+// = w, c = t, d = v.
 template <class T>
 __global__ void __launch_bounds__(256) k_bwd_gather(const int* __restrict__ dims, const int* __restrict__ ranks,
                                                     const long long* __restrict__ offX, const long long* __restrict__ offZ,
                                                     const long long* __restrict__ nrp, const long long* __restrict__ toff,
                                                     const T* __restrict__ x, const T* __restrict__ w,
                                                     const T* __restrict__ t, T* __restrict__ v, Strides ld, int nr) {
+  __shared__ long long to[TOFFS];
   const int i = blockIdx.x;
   const int M = dims[i], s = ranks[i];
-  for (int e = threadIdx.x; e < M * nr; e += 256) {
-    const int r = e % M, q = e / M;
-    T acc;
-    if (r < s) {
-      acc = w[offZ[i] + r + q * ld.b];
-    } else {
-      acc = x[offX[i] + r + q * ld.a];
-      acc -= sum_terms(t, toff, nrp[i], nrp[i + 1], (r - s) + q * ld.c);
-    }
-    v[offX[i] + r + q * ld.d] = acc;
+  if ((int)blockIdx.y * 256 >= M * nr) return;
+  const long long p0 = nrp[i], p1 = nrp[i + 1];
+  const bool staged = stage_toff(to, toff, p0, p1);
+  __syncthreads();
+  const int e = blockIdx.y * 256 + threadIdx.x;
+  if (e >= M * nr) return;
+  const int r = e % M, q = e / M;
+  T acc;
+  if (r < s) {
+    acc = w[offZ[i] + r + q * ld.b];
+  } else {
+    const long long off = (r - s) + q * ld.c;
+    acc = x[offX[i] + r + q * ld.a];
+    acc -= staged ? sum_terms_lds(t, to, (int)(p1 - p0), off) : sum_terms(t, toff, p0, p1, off);
   }
+  v[offX[i] + r + q * ld.d] = acc;
 }
 
 // Backward substitution: v_i = [w_i ; x_i[s:] - sum_near t_p], y_i = U_i v_i.
@@ -692,17 +851,14 @@ __global__ void __launch_bounds__(256) k_comb_bwd(const int* __restrict__ dims, 
                                                   const long long* __restrict__ offZ, const long long* __restrict__ nrp,
                                                   const long long* __restrict__ toff, const S* __restrict__ U,
                                                   const T* __restrict__ x, const T* __restrict__ w,
-                                                  const T* __restrict__ t, T* __restrict__ y, Strides ld, int mmax,
-                                                  int rows) {
+                                                  const T* __restrict__ t, T* __restrict__ y, Strides ld, int mmax) {
   __shared__ __align__(16) T red[lds_elems<T>()];
   __shared__ __align__(16) T vs[lds_elems<T>()];
   extern __shared__ __align__(16) unsigned char dsm[];
   T* xv = reinterpret_cast<T*>(dsm);  // mmax x NR
   const int i = blockIdx.x;
-  const int r0 = blockIdx.y * rows;  // this workgroup's rows of y_i: r0 .. r0 + rows - 1
   const int M = dims[i], s = ranks[i];
-  if (r0 >= M) return;
-  const int Mc = min(rows, M - r0);
+  if (M == 0) return;
   for (int e = threadIdx.x; e < M * NR; e += 256) {
     const int r = e % M, q = e / M;
     T acc;
@@ -715,9 +871,102 @@ __global__ void __launch_bounds__(256) k_comb_bwd(const int* __restrict__ dims, 
     xv[r + q * mmax] = acc;
   }
   __syncthreads();
-  T* yi = y + offX[i] + r0;
-  wg_gemv<T, S, V, NR>(U + offQ[i] + r0, M, Mc, M, [&](int c, int q) { return xv[c + q * mmax]; },
+  T* yi = y + offX[i];
+  wg_gemv<T, S, V, NR>(U + offQ[i], M, M, M, [&](int c, int q) { return xv[c + q * mmax]; },
                        [&](int r, int q, T v) { yi[r + q * ld.d] = v; }, red, vs);
+}
+
+// Downward pass of a level of few boxes, first half for several right-hand
+// sides: w_i += sum_far t_p in place, one element per thread.
+template <class T>
+__global__ void __launch_bounds__(256) k_gather_down(const int* __restrict__ ranks, const long long* __restrict__ offZ,
+                                                     const long long* __restrict__ frp, const long long* __restrict__ toff,
+                                                     T* __restrict__ w, long long ldw, const T* __restrict__ t,
+                                                     long long ldt, int nr) {
+  __shared__ long long to[TOFFS];
+  const int i = blockIdx.x, k = ranks[i];
+  if ((int)blockIdx.y * 256 >= k * nr) return;
+  const long long p0 = frp[i], p1 = frp[i + 1];
+  const bool staged = stage_toff(to, toff, p0, p1);
+  __syncthreads();
+  const int e = blockIdx.y * 256 + threadIdx.x;
+  if (e >= k * nr) return;
+  const int r = e % k, q = e / k;
+  T* x = w + offZ[i] + r + q * ldw;
+  const long long off = r + q * ldt;
+  *x += staged ? sum_terms_lds(t, to, (int)(p1 - p0), off) : sum_terms(t, toff, p0, p1, off);
+}
+
+// y_i = Q_i[:, :k] w_i (+ sum_near u_p at the leaf) for `rows` rows of a box, with
+// the far terms added to w_i while it is staged (GATHER) or before. Strides: a =
+// w, b = terms, d = y.
+template <class T, int V, int NR, bool GATHER>
+__global__ void __launch_bounds__(256) k_down_lat(const int* __restrict__ dims, const int* __restrict__ ranks,
+                                                  const long long* __restrict__ offQ, const long long* __restrict__ offX,
+                                                  const long long* __restrict__ offZ, const long long* __restrict__ frp,
+                                                  const long long* __restrict__ toffF, const long long* __restrict__ nrp,
+                                                  const long long* __restrict__ toffN, const T* __restrict__ Q,
+                                                  const T* __restrict__ w, const T* __restrict__ tF,
+                                                  const T* __restrict__ tN, T* __restrict__ y, Strides ld, int rows) {
+  __shared__ __align__(16) T xs[lat_elems<T>()];
+  __shared__ long long to[TOFFS];
+  const int i = blockIdx.x, r0 = blockIdx.y * rows, M = dims[i], k = ranks[i];
+  if (r0 >= M) return;
+  const int n = min(rows, M - r0);
+  const long long f0 = frp[i], f1 = frp[i + 1];
+  const long long n0 = tN ? nrp[i] : 0, n1 = tN ? nrp[i + 1] : 0;
+  const T* wi = w + offZ[i];
+  bool staged = false;
+  if constexpr (GATHER) staged = stage_toff(to, toffF, f0, f1);
+  auto stage = [&](int cb, int cn) {
+    stage_v<T, NR>(xs, cb, cn, [&](int c, int q) {
+      T s = wi[c + q * ld.a];
+      if constexpr (GATHER) {
+        const long long off = c + q * ld.b;
+        s += staged ? sum_terms_lds(tF, to, (int)(f1 - f0), off) : sum_terms(tF, toffF, f0, f1, off);
+      }
+      return s;
+    });
+  };
+  T* yi = y + offX[i] + r0;
+  auto emit = [&](int r, int q, T s) {
+    if (n1 > n0) s += sum_terms(tN, toffN, n0, n1, r0 + r + q * ld.b);
+    yi[r + q * ld.d] = s;
+  };
+  lat_gemv<T, T, V, NR>(Q + offQ[i] + r0, M, n, k, xs, stage, emit);
+}
+
+// Backward substitution of a level of few boxes: y_i = U_i v_i for `rows` rows of
+// a box, v_i = [w_i ; x_i[s:] - sum_near t_p] formed while it is staged (GATHER) or
+// read from v. Strides: a = x (or v), b = w, c = t, d = y.
+template <class T, class S, int V, int NR, bool GATHER>
+__global__ void __launch_bounds__(256) k_bwd_lat(const int* __restrict__ dims, const int* __restrict__ ranks,
+                                                 const long long* __restrict__ offQ, const long long* __restrict__ offX,
+                                                 const long long* __restrict__ offZ, const long long* __restrict__ nrp,
+                                                 const long long* __restrict__ toff, const S* __restrict__ U,
+                                                 const T* __restrict__ x, const T* __restrict__ w,
+                                                 const T* __restrict__ t, T* __restrict__ y, Strides ld, int rows) {
+  __shared__ __align__(16) T xs[lat_elems<T>()];
+  __shared__ long long to[TOFFS];
+  const int i = blockIdx.x, r0 = blockIdx.y * rows, M = dims[i], s = ranks[i];
+  if (r0 >= M) return;
+  const long long p0 = nrp[i], p1 = nrp[i + 1];
+  const T* xi = x + offX[i];
+  bool staged = false;
+  if constexpr (GATHER) staged = stage_toff(to, toff, p0, p1);
+  auto stage = [&](int cb, int cn) {
+    stage_v<T, NR>(xs, cb, cn, [&](int r, int q) {
+      if constexpr (!GATHER) return xi[r + q * ld.a];
+      if (r < s) return w[offZ[i] + r + q * ld.b];
+      T acc = xi[r + q * ld.a];
+      const long long off = (r - s) + q * ld.c;
+      acc -= staged ? sum_terms_lds(t, to, (int)(p1 - p0), off) : sum_terms(t, toff, p0, p1, off);
+      return acc;
+    });
+  };
+  T* yi = y + offX[i] + r0;
+  lat_gemv<T, S, V, NR>(U + offQ[i] + r0, M, min(rows, M - r0), M, xs, stage,
+                        [&](int r, int q, T v) { yi[r + q * ld.d] = v; });
 }
 
 __global__ void k_to_bf16(bf16_t* __restrict__ dst, const float* __restrict__ src, size_t n) {
@@ -749,7 +998,11 @@ void pair_jobs_append(std::vector<PairJob>& jobs, const std::vector<PairTask>& t
     MXG_REQUIRE(t.out + t.n <= nout && t.v + t.m <= nv, "pair task outside its vectors");
     MXG_REQUIRE(t.n == 0 || t.m == 0 || t.b + (long long)(t.m - 1) * t.ld + t.n <= nB, "pair task outside its matrix");
     const S* b = B + t.b;
-    const int vec = ((reinterpret_cast<uintptr_t>(b) % 16) == 0 && t.ld % W == 0 && t.n % W == 0) ? 1 : 0;
+    // vector loads of whole columns, the last vector of one perhaps past its n
+    // rows (what it holds there is dropped) but not past the matrix
+    const long long nw = (t.n + W - 1) / W * W;
+    const int vec = ((reinterpret_cast<uintptr_t>(b) % 16) == 0 && t.ld % W == 0 && nw <= t.ld &&
+                     (t.m == 0 || t.b + (long long)(t.m - 1) * t.ld + nw <= nB)) ? 1 : 0;
     const long long wave_bytes = std::is_same<S, bf16_t>::value ? 2 * WAVE_JOB_BYTES : WAVE_JOB_BYTES;
     const int wave = (t.n <= 64 * (vec ? W : 1) && (long long)t.n * t.m * (long long)sizeof(S) <= wave_bytes) ? 1 : 0;
     // the matrix cores take the aligned blocks stored in the compute type of
@@ -770,8 +1023,10 @@ template void pair_jobs_append<double, double>(std::vector<PairJob>&, const std:
 template void pair_jobs_append<float, bf16_t>(std::vector<PairJob>&, const std::vector<PairTask>&, const bf16_t*,
                                               long long, const float*, long long, long long, float*, long long, long long, bool);
 
-void pair_list_upload(PairList& pl, const std::vector<PairJob>& jobs, hipStream_t s) {
+void pair_list_upload(PairList& pl, const std::vector<PairJob>& jobs, hipStream_t s, bool few) {
   MXG_REQUIRE(jobs.size() < (1ull << 31), "pair list too long");
+  pl.few = few;
+  for (const PairJob& j : jobs) pl.few = pl.few && !j.mx && j.n <= LAT_ROWS;
   std::vector<PairJob> sorted;
   sorted.reserve(jobs.size());
   for (int mx : {1, 0}) {
@@ -801,6 +1056,18 @@ void pair_gemv(const PairList& pl, int nrhs, hipStream_t s) {
   for (int c0 = 0; c0 < nrhs;) {
     const int nr = batch_width(nrhs - c0);
     const dim3 b(256);
+    if (pl.few) {
+      const dim3 g((unsigned)pl.count);
+      switch (nr) {
+        case 8: hipLaunchKernelGGL((k_pair_gemv_lat<T, S, 8>), g, b, 0, s, pl.jobs.p, c0); break;
+        case 4: hipLaunchKernelGGL((k_pair_gemv_lat<T, S, 4>), g, b, 0, s, pl.jobs.p, c0); break;
+        case 2: hipLaunchKernelGGL((k_pair_gemv_lat<T, S, 2>), g, b, 0, s, pl.jobs.p, c0); break;
+        default: hipLaunchKernelGGL((k_pair_gemv_lat<T, S, 1>), g, b, 0, s, pl.jobs.p, c0); break;
+      }
+      MXG_HIP(hipGetLastError());
+      c0 += nr;
+      continue;
+    }
     if (gm > 0) {
       const dim3 g((unsigned)gm);
       switch (nr) {
@@ -829,9 +1096,51 @@ template void pair_gemv<double, double>(const PairList&, int, hipStream_t);
 template void pair_gemv<float, bf16_t>(const PairList&, int, hipStream_t);
 
 template <class T>
-void comb_down(const Level& Lv, bool vec, const long long* d_toffF, const long long* d_toffN, const T* Q, const T* w_in,
+void comb_down(const Level& Lv, bool vec, const long long* d_toffF, const long long* d_toffN, const T* Q, T* w_in,
                long long ldw, const T* tF, const T* tN, long long ldt, T* y, long long ldy, int nrhs, hipStream_t s) {
   if (Lv.nb == 0) return;
+  if ((size_t)Lv.nb < SPLIT_BELOW) {
+    const int rows = chunk_rows(Lv.nb);
+    const dim3 b(256), gp((unsigned)Lv.nb, ceil_div(std::max<long long>(Lv.maxM, 1), rows));
+    for (int c0 = 0; c0 < nrhs;) {
+      const int nr = batch_width(nrhs - c0);
+      const Strides ld{ldw, ldt, 0, ldy};
+      T* wi = w_in + c0 * ldw;
+      const T* f = tF + c0 * ldt;
+      const T* nn = tN ? tN + c0 * ldt : nullptr;
+      T* yo = y + c0 * ldy;
+      // the sums of the far terms: for one or two right-hand sides every
+      // workgroup of a box forms them (a launch less); for more, whose sums
+      // would take longer than a launch, they are formed once before
+      if (nr >= 4 && Lv.maxK > 0) {
+        hipLaunchKernelGGL(k_gather_down<T>, dim3((unsigned)Lv.nb, ceil_div(Lv.maxK * nr, 256)), b, 0, s, Lv.d_ranks.p,
+                           Lv.d_offZ.p, Lv.d_frp.p, d_toffF, wi, ldw, f, ldt, nr);
+        MXG_HIP(hipGetLastError());
+      }
+#define MXG_DOWN_LAT(VV, NN, GG)                                                                                      \
+  hipLaunchKernelGGL((k_down_lat<T, VV, NN, GG>), gp, b, 0, s, Lv.d_dims.p, Lv.d_ranks.p, Lv.d_offQ.p, Lv.d_offX.p,  \
+                     Lv.d_offZ.p, Lv.d_frp.p, d_toffF, Lv.d_nrp.p, d_toffN, Q, wi, f, nn, yo, ld, rows)
+      if (vec) {
+        switch (nr) {
+          case 8: MXG_DOWN_LAT(vwidth<T>(), 8, false); break;
+          case 4: MXG_DOWN_LAT(vwidth<T>(), 4, false); break;
+          case 2: MXG_DOWN_LAT(vwidth<T>(), 2, true); break;
+          default: MXG_DOWN_LAT(vwidth<T>(), 1, true); break;
+        }
+      } else {
+        switch (nr) {
+          case 8: MXG_DOWN_LAT(1, 8, false); break;
+          case 4: MXG_DOWN_LAT(1, 4, false); break;
+          case 2: MXG_DOWN_LAT(1, 2, true); break;
+          default: MXG_DOWN_LAT(1, 1, true); break;
+        }
+      }
+#undef MXG_DOWN_LAT
+      MXG_HIP(hipGetLastError());
+      c0 += nr;
+    }
+    return;
+  }
   const int kmax = (int)std::max<long long>(Lv.maxK, 1);
   const int fit = (int)(DYN_LDS_BYTES / ((size_t)kmax * sizeof(T)));
   MXG_REQUIRE(fit >= 1, "rank too large for the downward pass");
@@ -867,16 +1176,16 @@ void comb_down(const Level& Lv, bool vec, const long long* d_toffF, const long l
     c0 += nr;
   }
 }
-template void comb_down<float>(const Level&, bool, const long long*, const long long*, const float*, const float*,
+template void comb_down<float>(const Level&, bool, const long long*, const long long*, const float*, float*,
                                long long, const float*, const float*, long long, float*, long long, int, hipStream_t);
-template void comb_down<double>(const Level&, bool, const long long*, const long long*, const double*, const double*,
+template void comb_down<double>(const Level&, bool, const long long*, const long long*, const double*, double*,
                                 long long, const double*, const double*, long long, double*, long long, int, hipStream_t);
 
 template <class T>
 void comb_fwd(const Level& Lv, const long long* d_toff, const T* x, long long ldx, const T* t, long long ldt, T* z,
               long long ldz, int nrhs, hipStream_t s) {
   if (Lv.nb == 0 || Lv.lenZ == 0) return;
-  hipLaunchKernelGGL(k_comb_fwd<T>, dim3((unsigned)Lv.nb), dim3(256), 0, s, Lv.d_ranks.p, Lv.d_offX.p, Lv.d_offZ.p,
+  hipLaunchKernelGGL(k_comb_fwd<T>, dim3((unsigned)Lv.nb, ceil_div(Lv.maxK * nrhs, 256)), dim3(256), 0, s, Lv.d_ranks.p, Lv.d_offX.p, Lv.d_offZ.p,
                      Lv.d_nrp.p, d_toff, x, t, z, Strides{ldx, ldt, ldz, 0}, nrhs);
   MXG_HIP(hipGetLastError());
 }
@@ -889,7 +1198,7 @@ template <class T>
 void bwd_gather(const Level& Lv, const long long* d_toff, const T* x, long long ldx, const T* w, long long ldw, const T* t,
                 long long ldt, T* v, long long ldv, int nrhs, hipStream_t s) {
   if (Lv.nb == 0) return;
-  hipLaunchKernelGGL(k_bwd_gather<T>, dim3((unsigned)Lv.nb), dim3(256), 0, s, Lv.d_dims.p, Lv.d_ranks.p, Lv.d_offX.p,
+  hipLaunchKernelGGL(k_bwd_gather<T>, dim3((unsigned)Lv.nb, ceil_div(Lv.maxM * nrhs, 256)), dim3(256), 0, s, Lv.d_dims.p, Lv.d_ranks.p, Lv.d_offX.p,
                      Lv.d_offZ.p, Lv.d_nrp.p, d_toff, x, w, t, v, Strides{ldx, ldw, ldt, ldv}, nrhs);
   MXG_HIP(hipGetLastError());
 }
@@ -900,8 +1209,46 @@ template void bwd_gather<double>(const Level&, const long long*, const double*, 
 
 template <class T, class S>
 void comb_bwd(const Level& Lv, bool vec, const long long* d_toff, const S* U, const T* x, long long ldx, const T* w,
-              long long ldw, const T* t, long long ldt, T* y, long long ldy, int nrhs, hipStream_t s) {
+              long long ldw, const T* t, long long ldt, T* y, long long ldy, T* v, long long ldv, int nrhs, hipStream_t s) {
   if (Lv.nb == 0) return;
+  if ((size_t)Lv.nb < SPLIT_BELOW) {
+    const int rows = chunk_rows(Lv.nb);
+    const dim3 b(256), gp((unsigned)Lv.nb, ceil_div(std::max<long long>(Lv.maxM, 1), rows));
+    for (int c0 = 0; c0 < nrhs;) {
+      const int nr = batch_width(nrhs - c0);
+      const T* xi = x + c0 * ldx;
+      const T* wi = w + c0 * ldw;
+      const T* ti = t + c0 * ldt;
+      T* yo = y + c0 * ldy;
+      // as in comb_down: the box vectors formed by each workgroup, or once before
+      const bool once = nr >= 4;
+      if (once) bwd_gather<T>(Lv, d_toff, xi, ldx, wi, ldw, ti, ldt, v, ldv, nr, s);
+      const T* xv = once ? v : xi;
+      const Strides ld{once ? ldv : ldx, ldw, ldt, ldy};
+#define MXG_BWD_LAT(VV, NN, GG)                                                                                        \
+  hipLaunchKernelGGL((k_bwd_lat<T, S, VV, NN, GG>), gp, b, 0, s, Lv.d_dims.p, Lv.d_ranks.p, Lv.d_offQ.p, Lv.d_offX.p, \
+                     Lv.d_offZ.p, Lv.d_nrp.p, d_toff, U, xv, wi, ti, yo, ld, rows)
+      if (vec) {
+        switch (nr) {
+          case 8: MXG_BWD_LAT(vwidth<S>(), 8, false); break;
+          case 4: MXG_BWD_LAT(vwidth<S>(), 4, false); break;
+          case 2: MXG_BWD_LAT(vwidth<S>(), 2, true); break;
+          default: MXG_BWD_LAT(vwidth<S>(), 1, true); break;
+        }
+      } else {
+        switch (nr) {
+          case 8: MXG_BWD_LAT(1, 8, false); break;
+          case 4: MXG_BWD_LAT(1, 4, false); break;
+          case 2: MXG_BWD_LAT(1, 2, true); break;
+          default: MXG_BWD_LAT(1, 1, true); break;
+        }
+      }
+#undef MXG_BWD_LAT
+      MXG_HIP(hipGetLastError());
+      c0 += nr;
+    }
+    return;
+  }
   const int mmax = (int)std::max<long long>(Lv.maxM, 1);
   const int fit = (int)(DYN_LDS_BYTES / ((size_t)mmax * sizeof(T)));
   MXG_REQUIRE(fit >= 1, "box too large for the backward pass");
@@ -913,12 +1260,10 @@ void comb_bwd(const Level& Lv, bool vec, const long long* d_toff, const S* U, co
     const T* wi = w + c0 * ldw;
     const T* ti = t + c0 * ldt;
     T* yo = y + c0 * ldy;
-    // levels with few boxes split each box's product into chunks of rows
-    const int rows = (size_t)Lv.nb < SPLIT_BELOW ? SPLIT_ROWS : mmax;
-    const dim3 g((unsigned)Lv.nb, (unsigned)((mmax + rows - 1) / rows)), b(256);
+    const dim3 g((unsigned)Lv.nb), b(256);
 #define MXG_COMB_BWD(VV, NN)                                                                                          \
   hipLaunchKernelGGL((k_comb_bwd<T, S, VV, NN>), g, b, shm, s, Lv.d_dims.p, Lv.d_ranks.p, Lv.d_offQ.p, Lv.d_offX.p,  \
-                     Lv.d_offZ.p, Lv.d_nrp.p, d_toff, U, xi, wi, ti, yo, ld, mmax, rows)
+                     Lv.d_offZ.p, Lv.d_nrp.p, d_toff, U, xi, wi, ti, yo, ld, mmax)
     if (vec) {
       switch (nr) {
         case 8: MXG_COMB_BWD(vwidth<S>(), 8); break;
@@ -940,12 +1285,13 @@ void comb_bwd(const Level& Lv, bool vec, const long long* d_toff, const S* U, co
   }
 }
 template void comb_bwd<float, float>(const Level&, bool, const long long*, const float*, const float*, long long,
-                                     const float*, long long, const float*, long long, float*, long long, int, hipStream_t);
+                                     const float*, long long, const float*, long long, float*, long long, float*,
+                                     long long, int, hipStream_t);
 template void comb_bwd<double, double>(const Level&, bool, const long long*, const double*, const double*, long long,
-                                       const double*, long long, const double*, long long, double*, long long, int,
-                                       hipStream_t);
+                                       const double*, long long, const double*, long long, double*, long long,
+                                       double*, long long, int, hipStream_t);
 template void comb_bwd<float, bf16_t>(const Level&, bool, const long long*, const bf16_t*, const float*, long long,
-                                      const float*, long long, const float*, long long, float*, long long, int,
+                                      const float*, long long, const float*, long long, float*, long long, float*, long long, int,
                                       hipStream_t);
 
 void to_bf16(bf16_t* dst, const float* src, size_t n, hipStream_t s) {

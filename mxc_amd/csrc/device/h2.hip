@@ -17,7 +17,8 @@
 // The matvec (h2matrix.cpp:251-344) runs as lists of block products
 // (bgemv.hip): the upward pass level by level, the coupling products of
 // every level in one launch and, on the context's second stream beside
-// them, the leaf near products in one launch; then the downward per-box
+// them and after the leaf's upward products, the leaf near products in one
+// launch; then the downward per-box
 // sums level by level, of which only the leaf level waits for the near
 // products.
 #include "h2.hpp"
@@ -112,8 +113,9 @@ __global__ void __launch_bounds__(256) k_post(const PostTask* __restrict__ tasks
     }
 }
 
-// QT_i = Q_i[:, :k]^T (k x M, column major), the row-major basis the upward
-// pass streams with the block-sparse product kernel.
+// QT_i = Q_i[:, :k]^T (k x M, column major, leading dimension k rounded up to 4
+// for 16-byte loads), the row-major basis the upward pass streams with the
+// block-sparse product kernel.
 __global__ void __launch_bounds__(256) k_basis_transpose(const int* __restrict__ dims, const int* __restrict__ ranks,
                                                          const long long* __restrict__ offQ,
                                                          const long long* __restrict__ offQT, const double* __restrict__ Q,
@@ -122,9 +124,10 @@ __global__ void __launch_bounds__(256) k_basis_transpose(const int* __restrict__
   const int M = dims[i], k = ranks[i];
   const double* Qi = Q + offQ[i];
   double* Ti = QT + offQT[i];
+  const int ld = (k + 3) / 4 * 4;
   for (long long e = threadIdx.x; e < (long long)M * k; e += 256) {
     const int r = (int)(e % M), c = (int)(e / M);
-    Ti[c + (long long)r * k] = Qi[e];
+    Ti[c + (long long)r * ld] = Qi[e];
   }
 }
 
@@ -546,8 +549,8 @@ void basis_transpose(mxg_h2_s* h, Level& Lv) {
   hipStream_t s = h->ctx->stream;
   const long long nb = Lv.nb;
   Lv.offQT.assign(nb + 1, 0);
-  for (long long i = 0; i < nb; i++) Lv.offQT[i + 1] = Lv.offQT[i] + Lv.dims[i] * Lv.ranks[i];
-  Lv.QT.alloc(std::max<long long>(Lv.offQT[nb], 1));
+  for (long long i = 0; i < nb; i++) Lv.offQT[i + 1] = Lv.offQT[i] + Lv.dims[i] * ((Lv.ranks[i] + 3) / 4 * 4);
+  Lv.QT.alloc_zero(std::max<long long>(Lv.offQT[nb], 1), s);
   DevBuf<long long> d_offQT;
   d_offQT.upload(Lv.offQT, s);
   hipLaunchKernelGGL(k_basis_transpose, dim3((unsigned)nb), dim3(256), 0, s, Lv.d_dims.p, Lv.d_ranks.p, Lv.d_offQ.p, d_offQT.p,
@@ -594,7 +597,8 @@ void build_matvec_lists(mxg_h2_s* h, Level& Lv, bool leaf) {
   Lv.near_t.clear();
   for (long long i = 0; i < nb; i++)
     if (Lv.ranks[i] > 0)
-      Lv.up_t.push_back(PairTask{Lv.offQT[i], Lv.offX[i], Lv.offZ[i], (int)Lv.ranks[i], (int)Lv.dims[i], (int)Lv.ranks[i], 0});
+      Lv.up_t.push_back(PairTask{Lv.offQT[i], Lv.offX[i], Lv.offZ[i], (int)Lv.ranks[i], (int)Lv.dims[i],
+                                 (int)(Lv.ranks[i] + 3) / 4 * 4, 0});
   Lv.toffF.assign(Lv.frp[nb] + 1, 0);
   for (long long i = 0; i < nb; i++)
     for (long long p = Lv.frp[i]; p < Lv.frp[i + 1]; p++) {
@@ -689,6 +693,11 @@ void ensure_matvec_jobs(mxg_h2_s* h) {
   const MatvecTuning& tn = h->tune[pi];
   std::vector<PairJob> prod;
   std::vector<SymJob> prod_sym;
+  // the couplings of all levels are one launch: few of them are cut into rows
+  size_t nfar = 0;
+  for (long long l = 0; l <= L; l++) nfar += pi ? h->lv[l].far_t32.size() : h->lv[l].far_t.size();
+  const bool far_few = nfar < SPLIT_BELOW && !tn.matrix_cores;
+  auto far_rows = [&](const std::vector<PairTask>& t) { return far_few ? split_rows(t, chunk_rows(nfar)) : t; };
   for (long long l = 0; l <= L; l++) {
     Level& Lv = h->lv[l];
     std::vector<PairJob> up;
@@ -702,21 +711,22 @@ void ensure_matvec_jobs(mxg_h2_s* h) {
                            pi ? (long long)Lv.C32.n : (long long)Lv.C.n, Ops<T>::Z(h, l), Lv.lenZ, Lv.lenZ,
                            tb.p + Lv.tbaseF[pi], pi ? Lv.lenTF32 : Lv.lenTF, h->tlen[pi]);
       else
-        pair_jobs_append<T, T>(prod, pi ? Lv.far_t32 : Lv.far_t, Ops<T>::C(Lv),
+        pair_jobs_append<T, T>(prod, far_rows(pi ? Lv.far_t32 : Lv.far_t), Ops<T>::C(Lv),
                                pi ? (long long)Lv.C32.n : (long long)Lv.C.n, Ops<T>::Z(h, l), Lv.lenZ, Lv.lenZ,
                                tb.p + Lv.tbaseF[pi], pi ? Lv.lenTF32 : Lv.lenTF, h->tlen[pi], tn.matrix_cores != 0);
     }
-    pair_list_upload(Lv.up_pl[pi], up, s);
+    pair_list_upload(Lv.up_pl[pi], up, s, Lv.up_t.size() < SPLIT_BELOW);
   }
-  pair_list_upload(h->prod_pl[pi], prod, s);
+  pair_list_upload(h->prod_pl[pi], prod, s, far_few);
   sym_list_upload(h->prod_sym[pi], prod_sym, s);
   Level& Lf = h->lv[L];
   std::vector<PairJob> near;
   const bool near_sym = h->sym_near && tn.near_sym;
+  const bool near_few = Lf.near_t.size() < SPLIT_BELOW && !tn.matrix_cores;
   if (!near_sym)
-    pair_jobs_append<T, T>(near, Lf.near_t, Ops<T>::A(Lf), (long long)Lf.A.n, Ops<T>::x(h), h->n, h->n,
+    pair_jobs_append<T, T>(near, near_few ? split_rows(Lf.near_t, 2 * SPLIT_ROWS) : Lf.near_t, Ops<T>::A(Lf), (long long)Lf.A.n, Ops<T>::x(h), h->n, h->n,
                            tb.p + Lf.tbaseN[pi], Lf.lenTN, h->tlen[pi], tn.matrix_cores != 0);
-  pair_list_upload(h->near_pl[pi], near, s);
+  pair_list_upload(h->near_pl[pi], near, s, near_few);
   std::vector<SymJob> sym;
   if (near_sym)
     sym_jobs_append<T>(sym, Lf.near_sym_t, Ops<T>::A(Lf), (long long)Lf.A.n, Ops<T>::x(h), h->n, h->n,
@@ -761,20 +771,25 @@ void h2_matvec_levels(mxg_h2_s* h, T* y, long long ldy, int nrhs) {
   // beside the upward pass and the far terms, which leave most of the GPU idle
   hipStream_t sa = h->ctx->aux;
   ProfScope whole(h->ctx, f64 ? MXG_PROF_MATVEC_FP64 : MXG_PROF_MATVEC_FP32);
-  MXG_HIP(hipEventRecord(h->ctx->fork, s));
-  MXG_HIP(hipStreamWaitEvent(sa, h->ctx->fork, 0));
-  {
-    ProfScope prof(h->ctx, f64 ? MXG_PROF_MATVEC_LEAF_FP64 : MXG_PROF_MATVEC_LEAF_FP32, sa);
-    // one of the two lists is empty
-    sym_gemv<T>(h->near_sym[pi], nrhs, sa);
-    pair_gemv<T, T>(h->near_pl[pi], nrhs, sa);
-  }
-  MXG_HIP(hipEventRecord(h->ctx->join, sa));
-  // upward pass: z_i = Q_i[:, :k]^T x_i
+  // upward pass: z_i = Q_i[:, :k]^T x_i. Its leaf level goes first and alone: it
+  // is bound by bytes, and beside the near products it would have the few CUs
+  // left to the context stream (N = 131072, 8 right-hand sides: 79 us there, 21
+  // alone)
   for (long long l = L; l >= 0; l--) {
-    if (h->lv[l].lenZ == 0) continue;
-    ProfScope prof(h->ctx, MXG_PROF_MATVEC_UPPER);
-    pair_gemv<T, T>(h->lv[l].up_pl[pi], nrhs, s);
+    if (h->lv[l].lenZ > 0) {
+      ProfScope prof(h->ctx, MXG_PROF_MATVEC_UPPER);
+      pair_gemv<T, T>(h->lv[l].up_pl[pi], nrhs, s);
+    }
+    if (l == L) {
+      MXG_HIP(hipEventRecord(h->ctx->fork, s));
+      MXG_HIP(hipStreamWaitEvent(sa, h->ctx->fork, 0));
+      ProfScope prof(h->ctx, f64 ? MXG_PROF_MATVEC_LEAF_FP64 : MXG_PROF_MATVEC_LEAF_FP32, sa);
+      // one of the two lists is empty
+      sym_gemv<T>(h->near_sym[pi], nrhs, sa);
+      pair_gemv<T, T>(h->near_pl[pi], nrhs, sa);
+      prof.end();
+      MXG_HIP(hipEventRecord(h->ctx->join, sa));
+    }
   }
   // every far term of every level, one launch
   {

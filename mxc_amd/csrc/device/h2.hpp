@@ -39,9 +39,12 @@ inline std::vector<PairTask> split_rows(const std::vector<PairTask>& tasks, int 
 // levels with fewer blocks than this get their rows split (chunks of 32)
 constexpr size_t SPLIT_BELOW = 1024;
 constexpr int SPLIT_ROWS = 32;
-inline std::vector<PairTask> spread(const std::vector<PairTask>& tasks, size_t below = SPLIT_BELOW,
-                                    int rows = SPLIT_ROWS) {
-  return tasks.size() < below ? split_rows(tasks, rows) : tasks;
+// rows of a chunk for that many blocks: from 256 blocks on, chunks of 32 would be
+// more workgroups than the GPU holds at a time, each staging the same inputs
+// (N = 131072, bfloat16 factors of 512 boxes, 8 right-hand sides: 37 -> 25 us)
+inline int chunk_rows(size_t blocks) { return blocks >= 256 ? 2 * SPLIT_ROWS : SPLIT_ROWS; }
+inline std::vector<PairTask> spread(const std::vector<PairTask>& tasks, size_t below = SPLIT_BELOW, int rows = 0) {
+  return tasks.size() < below ? split_rows(tasks, rows ? rows : chunk_rows(tasks.size())) : tasks;
 }
 
 // Launch shapes of one precision's matvec, chosen by mxg_h2_autotune: the
@@ -104,6 +107,7 @@ struct PairList {
   long long count = 0;                   // all jobs
   long long count_mx = 0, nbig_mx = 0;   // jobs [0, count_mx), the first nbig_mx workgroup-sized
   long long nbig = 0;                    // workgroup-sized jobs among [count_mx, count)
+  bool few = false;                      // a list of few blocks: one workgroup per job, deep loads
 };
 
 struct Level {
@@ -217,7 +221,9 @@ typedef unsigned short bf16_t;
 template <class T, class S>
 void pair_jobs_append(std::vector<PairJob>& jobs, const std::vector<PairTask>& tasks, const S* B, long long nB, const T* v,
                       long long nv, long long ldv, T* out, long long nout, long long ldo, bool matrix_cores = false);
-void pair_list_upload(PairList& pl, const std::vector<PairJob>& jobs, hipStream_t s);
+// few: the list comes from fewer than SPLIT_BELOW blocks, cut into chunks of
+// rows; it runs as one workgroup per job when no job has more than 64 rows
+void pair_list_upload(PairList& pl, const std::vector<PairJob>& jobs, hipStream_t s, bool few = false);
 // out[r + k ldo] = sum_c B[r + c*ld] v[c + k ldv] for every job and the
 // right-hand sides k < nrhs (<= MAX_RHS), one workgroup per job, blocks
 // stored as S, arithmetic in T
@@ -236,9 +242,10 @@ void sym_gemv(const SymList& sl, int nrhs, hipStream_t s);
 // FP32 -> bfloat16, round to nearest even
 void to_bf16(bf16_t* dst, const float* src, size_t n, hipStream_t s);
 // w_i = w_in_i + sum_far tF, y_i = Q_i[:, :k] w_i (+ sum_near tN when tN !=
-// nullptr); ld*: strides between right-hand sides (tF and tN share ldt)
+// nullptr); ld*: strides between right-hand sides (tF and tN share ldt); w_in
+// may be overwritten with w
 template <class T>
-void comb_down(const Level& Lv, bool vec, const long long* d_toffF, const long long* d_toffN, const T* Q, const T* w_in,
+void comb_down(const Level& Lv, bool vec, const long long* d_toffF, const long long* d_toffN, const T* Q, T* w_in,
                long long ldw, const T* tF, const T* tN, long long ldt, T* y, long long ldy, int nrhs, hipStream_t s);
 // z_i = x_i[:s] - sum_near t
 template <class T>
@@ -248,8 +255,9 @@ void comb_fwd(const Level& Lv, const long long* d_toff, const T* x, long long ld
 template <class T>
 void bwd_gather(const Level& Lv, const long long* d_toff, const T* x, long long ldx, const T* w, long long ldw, const T* t,
                 long long ldt, T* v, long long ldv, int nrhs, hipStream_t s);
-// y_i = U_i [w_i ; x_i[s:] - sum_near t], U stored as S
+// y_i = U_i [w_i ; x_i[s:] - sum_near t], U stored as S; v: scratch for the box
+// vectors, as x (stride ldv)
 template <class T, class S>
 void comb_bwd(const Level& Lv, bool vec, const long long* d_toff, const S* U, const T* x, long long ldx, const T* w,
-              long long ldw, const T* t, long long ldt, T* y, long long ldy, int nrhs, hipStream_t s);
+              long long ldw, const T* t, long long ldt, T* y, long long ldy, T* v, long long ldv, int nrhs, hipStream_t s);
 }  // namespace mxg

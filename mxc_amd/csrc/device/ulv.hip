@@ -300,15 +300,15 @@ struct UlvImpl : UlvBase {
     pair_jobs_append<T, S>(jv, spread(vt), Vstore(F), H.offQ[nb], y, ylen, ylen, F.X.p, lx, lx);
     pair_jobs_append<T, S>(jf, spread(ft), Astore(F), (long long)F.A.n, F.X.p, lx, lx, tbuf.p, tlen, tlen);
     pair_jobs_append<T, S>(jb, spread(bt), Astore(F), (long long)F.A.n, F.Z.p, lz, lz, tbuf.p, tlen, tlen);
-    pair_list_upload(F.v_pl, jv, s);
-    pair_list_upload(F.fwd_pl, jf, s);
-    pair_list_upload(F.bwd_pl, jb, s);
+    pair_list_upload(F.v_pl, jv, s, vt.size() < SPLIT_BELOW);
+    pair_list_upload(F.fwd_pl, jf, s, ft.size() < SPLIT_BELOW);
+    pair_list_upload(F.bwd_pl, jb, s, bt.size() < SPLIT_BELOW);
     if (l == h->L) {
       // the leaf's U products as their own launch: a 256 x 256 bfloat16 box
       // factor is then one wave's job rather than one workgroup's
       std::vector<PairJob> ju;
       pair_jobs_append<T, S>(ju, spread(vt), Ustore(F), H.offQ[nb], ubuf.p, lx, lx, vin.p, h->n, h->n);
-      pair_list_upload(F.u_pl, ju, s);
+      pair_list_upload(F.u_pl, ju, s, vt.size() < SPLIT_BELOW);
     }
     F.d_toffU.upload(toffU, s);
     F.d_toffB.upload(toffB, s);
@@ -553,7 +553,7 @@ struct UlvImpl : UlvBase {
           bwd_gather<T>(H, F.d_toffB.p, F.X.p, lx, F.Z.p, lz, tbuf.p, tlen, ubuf.p, lx, nr, s);
           pair_gemv<T, S>(F.u_pl, nr, s);
         } else {
-          comb_bwd<T, S>(H, F.vecM, F.d_toffB.p, Ustore(F), F.X.p, lx, F.Z.p, lz, tbuf.p, tlen, out, lo, nr, s);
+          comb_bwd<T, S>(H, F.vecM, F.d_toffB.p, Ustore(F), F.X.p, lx, F.Z.p, lz, tbuf.p, tlen, out, lo, ubuf.p, lx, nr, s);
         }
       }
       whole.end();
