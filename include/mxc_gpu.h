@@ -60,7 +60,8 @@ const char* mxg_last_error(void);
 /* HIP stream of the context (a hipStream_t) */
 void* mxg_stream(mxg_ctx_t ctx);
 /* free and total device memory of the context's GPU (hipMemGetInfo), for
- * callers that admit work by its memory footprint */
+ * callers that admit work by its memory footprint. Memory that contexts keep
+ * for reuse counts as free: an allocation that needs it gets it. */
 int mxg_mem_info(mxg_ctx_t ctx, size_t* free_bytes, size_t* total_bytes);
 
 /* device memory for callers without an allocator of their own */

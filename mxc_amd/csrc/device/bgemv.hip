@@ -1329,6 +1329,7 @@ extern "C" int mxg_block_gemv(mxg_ctx_t ctx, int storage, long long n, long long
     MXG_REQUIRE(nrhs >= 1 && nrhs <= MAX_RHS, "nrhs must be 1..8");
     MXG_REQUIRE(d_B && d_X && d_Y, "null pointer");
     MXG_HIP(hipSetDevice(ctx->device));
+    PoolScope pool(ctx->pool);
     if (storage == MXG_FP64)
       one_block<double, double>(ctx, n, m, d_B, ldb, d_X, ldx, d_Y, ldy, (int)nrhs, matrix_cores != 0);
     else if (storage == MXG_FP32)

@@ -1,6 +1,9 @@
 // Context, memory helpers and error reporting of the device layer.
 // Replaces gpu_handles.cu:5-12 (device selection) and :54-71 (streams and
 // handles); there are no BLAS/SPARSE handles: every kernel is our own.
+#include <algorithm>
+#include <atomic>
+
 #include "common.hpp"
 
 namespace mxg {
@@ -8,6 +11,116 @@ namespace {
 thread_local std::string g_last_error;
 }
 void set_last_error(const std::string& msg) { g_last_error = msg; }
+
+// ---- device memory pools ----
+namespace {
+struct Pools {
+  std::mutex mu;  // taken before a pool's own
+  std::vector<DevPool*> all;
+  std::atomic<size_t> kept{0};  // bytes kept by all pools
+  std::atomic<size_t> most{0};  // and at most
+};
+// never destroyed: buffers may be released while the process ends
+Pools& pools() {
+  static Pools* p = new Pools;
+  return *p;
+}
+void trim_pools() {
+  Pools& P = pools();
+  std::lock_guard<std::mutex> lk(P.mu);
+  for (DevPool* p : P.all) p->trim();
+}
+}  // namespace
+
+hipError_t device_malloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess && pools().kept.load() > 0) {
+    (void)hipGetLastError();
+    trim_pools();
+    e = hipMalloc(p, bytes);
+  }
+  return e;
+}
+
+DevPool::DevPool(int device) : device_(device) {
+  size_t free_b = 0, total = 0;
+  if (hipMemGetInfo(&free_b, &total) != hipSuccess) total = 0;
+  Pools& P = pools();
+  std::lock_guard<std::mutex> lk(P.mu);
+  P.most = total / 32;
+  P.all.push_back(this);
+}
+
+DevPool::~DevPool() {
+  Pools& P = pools();
+  {
+    std::lock_guard<std::mutex> lk(P.mu);
+    P.all.erase(std::find(P.all.begin(), P.all.end(), this));
+  }
+  trim();
+}
+
+void* DevPool::take(size_t bytes, size_t* cap) {
+  // whole 512 bytes, above a megabyte whole 64 KB: arrays whose sizes differ
+  // little from one object to the next share blocks
+  const size_t unit = bytes > (size_t(1) << 20) ? size_t(65536) : size_t(512);
+  const size_t need = (bytes + unit - 1) / unit * unit;
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    auto it = free_.lower_bound(need);
+    if (it != free_.end() && it->first <= need + need / 4 + 4096) {
+      void* p = it->second;
+      *cap = it->first;
+      kept_ -= it->first;
+      pools().kept -= it->first;
+      free_.erase(it);
+      return p;
+    }
+  }
+  void* p = nullptr;
+  const hipError_t e = device_malloc(&p, need);
+  if (e != hipSuccess)
+    throw Error(MXG_ERR_NOMEM, "hipMalloc of " + std::to_string(need) + " bytes failed: " + hipGetErrorString(e));
+  *cap = need;
+  return p;
+}
+
+void DevPool::give(void* p, size_t cap) {
+  Pools& P = pools();
+  if (P.kept.fetch_add(cap) + cap > P.most.load()) {
+    P.kept -= cap;
+    (void)hipFree(p);
+    return;
+  }
+  std::lock_guard<std::mutex> lk(mu_);
+  kept_ += cap;
+  free_.emplace(cap, p);
+}
+
+void DevPool::trim() {
+  std::lock_guard<std::mutex> lk(mu_);
+  for (auto& b : free_) (void)hipFree(b.second);
+  pools().kept -= kept_;
+  kept_ = 0;
+  free_.clear();
+}
+
+size_t DevPool::kept_on(int device) {
+  Pools& P = pools();
+  std::lock_guard<std::mutex> lk(P.mu);
+  size_t sum = 0;
+  for (DevPool* p : P.all)
+    if (p->device_ == device) {
+      std::lock_guard<std::mutex> lp(p->mu_);
+      sum += p->kept_;
+    }
+  return sum;
+}
+
+std::shared_ptr<DevPool>& DevPool::current() {
+  static thread_local std::shared_ptr<DevPool> p;
+  return p;
+}
 
 namespace {
 hipEvent_t take_event(mxg_ctx_s* c) {
@@ -112,6 +225,7 @@ int mxg_init(int device, mxg_ctx_t* ctx) {
       throw Error(MXG_ERR_HIP, std::string("stream or event creation failed: ") + hipGetErrorString(e));
     }
     try {
+      c->pool = std::make_shared<DevPool>(device);
       dense_scratch_setup(device);
     } catch (...) {
       (void)hipEventDestroy(c->join);
@@ -187,6 +301,7 @@ int mxg_mem_info(mxg_ctx_t ctx, size_t* free_bytes, size_t* total_bytes) {
     MXG_REQUIRE(ctx && free_bytes && total_bytes, "null argument");
     MXG_HIP(hipSetDevice(ctx->device));
     MXG_HIP(hipMemGetInfo(free_bytes, total_bytes));
+    *free_bytes += DevPool::kept_on(ctx->device);
   });
 }
 
@@ -203,7 +318,7 @@ int mxg_malloc(mxg_ctx_t ctx, size_t bytes, void** d_ptr) {
     MXG_HIP(hipSetDevice(ctx->device));
     *d_ptr = nullptr;
     if (bytes == 0) return;
-    hipError_t e = hipMalloc(d_ptr, bytes);
+    hipError_t e = device_malloc(d_ptr, bytes);
     if (e != hipSuccess) throw Error(MXG_ERR_NOMEM, std::string("hipMalloc failed: ") + hipGetErrorString(e));
   });
 }

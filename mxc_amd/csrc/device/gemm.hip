@@ -340,6 +340,7 @@ extern "C" int mxg_gemm(mxg_ctx_t ctx, int precision, int ta, int tb, long long 
     MXG_REQUIRE(lda >= std::max<long long>(ta ? k : m, 1) && ldb >= std::max<long long>(tb ? n : k, 1), "lda/ldb too small");
     if (m == 0 || n == 0) return;
     MXG_REQUIRE(d_C && (k == 0 || (d_A && d_B)), "null pointer");
+    PoolScope pool(ctx->pool);
     if (precision == MXG_FP64)
       one_gemm<double>(ctx, ta, tb, m, n, k, alpha, d_A, lda, d_B, ldb, beta, d_C, ldc);
     else if (precision == MXG_FP32)

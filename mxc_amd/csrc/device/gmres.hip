@@ -597,6 +597,7 @@ extern "C" int mxg_gmres(mxg_h2_t A, mxg_ulv_t M, const mxg_gmres_opts_t* o, con
     check_opts(A, M, o);
     MXG_REQUIRE(d_b && d_x && resid, "null argument");
     MXG_HIP(hipSetDevice(A->ctx->device));
+    PoolScope pool(A->ctx->pool);
     gmres_batch(A, M, o, 1, d_b, A->n, d_x, A->n, resid, iters_out, inner_out);
   });
 }
@@ -610,6 +611,7 @@ extern "C" int mxg_gmres_batch(mxg_h2_t A, mxg_ulv_t M, const mxg_gmres_opts_t* 
     MXG_REQUIRE(nrhs >= 1 && nrhs <= 64, "nrhs out of range (1..64)");
     MXG_REQUIRE(ldb >= A->n && ldx >= A->n, "bad leading dimensions");
     MXG_HIP(hipSetDevice(A->ctx->device));
+    PoolScope pool(A->ctx->pool);
     gmres_batch(A, M, o, (int)nrhs, d_b, ldb, d_x, ldx, resid, iters_out, inner_out);
   });
 }

@@ -1132,6 +1132,7 @@ int mxg_h2_create(mxg_ctx_t ctx, mxg_kernel_t k, const double* bodies, long long
     MXG_REQUIRE(levels >= 0 && levels < 31 && (1ll << levels) <= nbodies, "levels out of range");
     MXG_REQUIRE(k.id >= MXG_KERNEL_LAPLACE && k.id <= MXG_KERNEL_GAUSSIAN, "unknown kernel id");
     MXG_HIP(hipSetDevice(ctx->device));
+    PoolScope pool(ctx->pool);
     auto* h = new mxg_h2_s();
     try {
       h->ctx = ctx;
@@ -1172,6 +1173,7 @@ void construct_level(mxg_h2_t h, long long l, long long nb, const long long* dim
     MXG_REQUIRE(l >= 0 && l <= h->L, "level out of range");
     MXG_REQUIRE(l < h->L || leaf_begin, "leaf level needs leaf_begin");
     MXG_HIP(hipSetDevice(h->ctx->device));
+    PoolScope pool(h->ctx->pool);
     hipStream_t s = h->ctx->stream;
     level_structure(h, l, nb, dims, near_rp, near_col, far_rp, far_col);
     Level& Lv = h->lv[l];
@@ -1238,6 +1240,7 @@ int mxg_h2_construct_level(mxg_h2_t h, long long l, long long nb, const long lon
     MXG_REQUIRE(h && dims && ranks_out, "null argument");
     MXG_REQUIRE(l >= 0 && l <= h->L, "level out of range");
     MXG_HIP(hipSetDevice(h->ctx->device));
+    PoolScope pool(h->ctx->pool);
     FarRows fr;
     if (l > 0) far_rows_explicit(h, nb, far_off, far_idx, fr);
     else far_rows_explicit(h, nb, nullptr, nullptr, fr);
@@ -1254,6 +1257,7 @@ int mxg_h2_construct_level_runs(mxg_h2_t h, long long l, long long nb, const lon
     MXG_REQUIRE(l >= 0 && l <= h->L, "level out of range");
     MXG_REQUIRE(!far_run_off || far_runs || far_run_off[nb] == far_run_off[0], "null far runs");
     MXG_HIP(hipSetDevice(h->ctx->device));
+    PoolScope pool(h->ctx->pool);
     FarRows fr;
     far_rows_runs(h, nb, l > 0 ? far_run_off : nullptr, far_runs, fr);
     construct_level(h, l, nb, dims, leaf_begin, near_rp, near_col, far_rp, far_col, fr, tol, maxrank, orth, ranks_out);
@@ -1267,6 +1271,7 @@ int mxg_h2_define_level(mxg_h2_t h, long long l, long long nb, const long long* 
     MXG_REQUIRE(h && dims && ranks && near_rp && far_rp, "null argument");
     MXG_REQUIRE(l >= 0 && l <= h->L, "level out of range");
     MXG_HIP(hipSetDevice(h->ctx->device));
+    PoolScope pool(h->ctx->pool);
     hipStream_t s = h->ctx->stream;
     for (long long i = 0; i < nb; i++) MXG_REQUIRE(ranks[i] >= 0 && ranks[i] <= dims[i], "rank out of range (0..dim)");
     if (l == 0) for (long long i = 0; i < nb; i++) MXG_REQUIRE(ranks[i] == 0, "the root has rank 0");
@@ -1336,6 +1341,7 @@ int mxg_h2_upload(mxg_h2_t h, long long l, int what, const double* src, long lon
     const long long n = mxg_h2_level_size(h, l, what);
     MXG_REQUIRE(n >= 0 && count == n, "count does not match the level size");
     MXG_HIP(hipSetDevice(h->ctx->device));
+    PoolScope pool(h->ctx->pool);
     if (n == 0) return;
     Level& Lv = h->lv[l];
     hipStream_t s = h->ctx->stream;
@@ -1377,6 +1383,7 @@ int mxg_h2_autotune(mxg_h2_t h, int precision, long long nrhs, int reps, double*
     MXG_REQUIRE(nrhs >= 1 && nrhs <= MAX_RHS && reps >= 1 && reps <= 1000, "nrhs must be 1..8 and reps 1..1000");
     for (long long l = 0; l <= h->L; l++) MXG_REQUIRE(h->lv[l].built, "H2 matrix not fully constructed");
     MXG_HIP(hipSetDevice(h->ctx->device));
+    PoolScope pool(h->ctx->pool);
     if (precision == MXG_FP32) {
       make_shadow32(h);
       *best_ms = autotune<float>(h, (int)nrhs, reps);
@@ -1420,6 +1427,7 @@ int mxg_h2_matvec(mxg_h2_t h, const double* d_x, double* d_y, long long nrhs, lo
     MXG_REQUIRE(h && d_x && d_y, "null argument");
     MXG_REQUIRE(nrhs >= 1 && ld >= h->n, "bad nrhs/ld");
     MXG_HIP(hipSetDevice(h->ctx->device));
+    PoolScope pool(h->ctx->pool);
     h2_apply(h, d_x, ld, d_y, ld, nrhs, precision);
     MXG_HIP(hipStreamSynchronize(h->ctx->stream));
   });

@@ -242,6 +242,7 @@ int mxg_gen_block(mxg_ctx_t ctx, mxg_kernel_t k, long long m, long long n, const
     MXG_REQUIRE(m < (1ll << 31) && n < (1ll << 31) && lda < (1ll << 31), "block too large");
     if (m == 0 || n == 0) return;
     MXG_REQUIRE(d_bi && d_bj && d_A, "null pointer");
+    PoolScope pool(ctx->pool);
     // Points of the two sides are separate arrays: stage them as one body array.
     DevBuf<double> pts;
     pts.alloc(3 * (size_t)(m + n));
@@ -262,6 +263,7 @@ int mxg_dense_matvec_batch(mxg_ctx_t ctx, mxg_kernel_t k, const double* d_bodies
     MXG_REQUIRE(ldx >= n && ldy >= n, "bad leading dimensions");
     const int nchunks = (int)ceil_div(n, DM_CHUNK);
     MXG_REQUIRE(ceil_div(n, DM_ROWS) < (1u << 31) && nchunks < 65536, "dense check size too large");
+    PoolScope pool(ctx->pool);
     DevBuf<double> part;
     part.alloc((size_t)nchunks * n * std::min<long long>(nrhs, 8));
     for (long long c0 = 0; c0 < nrhs;) {

@@ -591,6 +591,7 @@ int mxg_ulv_create(mxg_h2_t h, int precision, mxg_ulv_t* out) {
     MXG_REQUIRE(precision == MXG_FP64 || precision == MXG_FP32 || precision == MXG_BF16 || precision == MXG_BF16_SCHUR,
                 "unknown precision");
     MXG_HIP(hipSetDevice(h->ctx->device));
+    PoolScope pool(h->ctx->pool);
     auto f = std::make_unique<mxg_ulv_s>();
     f->h = h;
     f->precision = precision;
@@ -632,6 +633,7 @@ int mxg_ulv_create_batch(const mxg_h2_t* hs, long long count, int precision, mxg
       for (long long q = 0; q < p; q++) MXG_REQUIRE(hs[q] != hs[p], "a matrix appears twice in the batch");
     }
     MXG_HIP(hipSetDevice(ctx->device));
+    PoolScope pool(ctx->pool);
     std::vector<std::unique_ptr<mxg_ulv_s>> fs(count);
     auto run = [&](auto* tag) {
       using Impl = std::remove_pointer_t<decltype(tag)>;
@@ -687,6 +689,7 @@ int mxg_ulv_solve(mxg_ulv_t f, double* d_x, long long nrhs, long long ld) {
     MXG_REQUIRE(f && d_x, "null argument");
     MXG_REQUIRE(nrhs >= 1 && ld >= f->h->n, "bad nrhs/ld");
     MXG_HIP(hipSetDevice(f->h->ctx->device));
+    PoolScope pool(f->h->ctx->pool);
     f->impl->solve(d_x, ld, nrhs);
     MXG_HIP(hipStreamSynchronize(f->h->ctx->stream));
   });

@@ -1,0 +1,71 @@
+"""Device memory kept on a context for its later objects: contexts at work in
+several threads at once, and memory given back when a context goes."""
+import ctypes as C
+import threading
+
+import numpy as np
+import pytest
+
+import oracle_lib as O
+from mxc_amd import _native as N
+from mxc_amd.device import Context
+from mxc_amd.solver import H2, Problem
+
+pytestmark = pytest.mark.gpu
+
+
+def work(ctx, n, seed):
+    prob = Problem(ctx, O.cube_points(n, seed), 128)
+    out = []
+    for rank in (40, 64, 40):
+        M = H2.preconditioner(prob, rank, 500)
+        for prec in (N.MXG_FP64, N.MXG_FP32):
+            M.factorize(prec)
+            d = ctx.array(O.uniform_vec(n, -1, 1, 7))
+            M.precondition(d)
+            out.append(d.download())
+        M.close()
+    A = H2.operator(prob, 1e-9, 500)
+    x, y = ctx.array(O.uniform_vec(n, -1, 1, 8)), ctx.zeros(n)
+    A.matvec(x, y)
+    out.append(y.download())
+    A.close()
+    prob.close()
+    return out
+
+
+@pytest.mark.timeout(120)
+def test_contexts_in_threads(ctx):
+    sizes = [(900, 1), (2500, 2), (4096, 3), (5000, 4)]
+    alone = [work(ctx, n, s) for n, s in sizes]
+    got = [None] * len(sizes)
+
+    def run(k):
+        c = Context(0)
+        got[k] = work(c, *sizes[k])
+        c.close()
+    threads = [threading.Thread(target=run, args=(k,)) for k in range(len(sizes))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for a, g in zip(alone, got):
+        assert g is not None and all(np.array_equal(u, v) for u, v in zip(a, g))
+
+
+def test_memory_goes_back_with_the_context():
+    hip = C.CDLL("libamdhip64.so")
+
+    def free():
+        f, t = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+    Context(0).close()
+    before = free()
+    for _ in range(2):
+        c = Context(0)
+        work(c, 8192, 5)
+        # kept memory counts as free (the factorizations' own scratch does not)
+        assert c.mem_info()[0] >= free()
+        c.close()
+    assert before - free() < (64 << 20)
