@@ -292,6 +292,23 @@ inline unsigned ceil_div(long long a, long long b) { return (unsigned)((a + b - 
 
 // ---- device helpers ----
 
+// A pointer that a kernel read from a task descriptor, with what the compiler
+// cannot know: that it points into device memory. Without it every access is
+// a flat one, which counts as an LDS access too: it waits in order behind LDS
+// reads and they behind it, so that no load stays in flight across them.
+template <class T>
+__device__ inline T* in_global(T* p) {
+  return (T*)(__attribute__((address_space(1))) T*)(unsigned long long)p;
+}
+
+// A pointer to descriptors that no kernel in flight writes: at an address that
+// a whole wave shares they are read by scalar loads, which do not wait for
+// the vector loads in flight.
+template <class T>
+__device__ inline const T* in_constant(const T* p) {
+  return (const T*)(const __attribute__((address_space(4))) T*)(unsigned long long)p;
+}
+
 __device__ inline double wave_sum(double v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
