@@ -26,6 +26,14 @@
 namespace mxg {
 namespace {
 
+__device__ inline PairJob read_job(const PairJob* __restrict__ jobs, long long i) {
+  PairJob t = in_constant(jobs)[i];
+  t.B = in_global(t.B);
+  t.v = in_global(t.v);
+  t.out = in_global(t.out);
+  return t;
+}
+
 template <class T, int V> struct Vec { typedef T type __attribute__((ext_vector_type(V))); };
 template <> struct Vec<float, 1> { typedef float type; };
 template <> struct Vec<double, 1> { typedef double type; };
@@ -546,11 +554,11 @@ __global__ void __launch_bounds__(256) k_pair_gemv_mx(const PairJob* __restrict_
     const int wave = wave_id();
     const long long j = nbig + ((long long)blockIdx.x - nbig) * 4 + wave;
     if (j >= count) return;
-    wave_gemv_mfma<T, S, NR>(jobs[j], c0, vs + wave * (lds_elems<T>() / 4));
+    wave_gemv_mfma<T, S, NR>(read_job(jobs, j), c0, vs + wave * (lds_elems<T>() / 4));
     return;
   }
   if constexpr (std::is_same<T, S>::value) {
-    const PairJob t = jobs[blockIdx.x];
+    const PairJob t = read_job(jobs, blockIdx.x);
     const T* vb = static_cast<const T*>(t.v) + (long long)c0 * t.ldv;
     T* ob = static_cast<T*>(t.out) + (long long)c0 * t.ldo;
     wg_gemv_mfma<T, NR>(static_cast<const T*>(t.B), t.ld, t.n, t.m, vb, t.ldv, ob, t.ldo, vs);
@@ -569,7 +577,7 @@ __global__ void __launch_bounds__(256) k_pair_gemv(const PairJob* __restrict__ j
     const int wave = wave_id();
     const long long j = nbig + ((long long)blockIdx.x - nbig) * 4 + wave;
     if (j >= count) return;
-    const PairJob t = jobs[j];
+    const PairJob t = read_job(jobs, j);
     T* vw = vs + wave * (lds_elems<T>() / 4);
     if (t.vec)
       wave_gemv<T, S, VW, NR>(t, c0, vw);
@@ -577,7 +585,7 @@ __global__ void __launch_bounds__(256) k_pair_gemv(const PairJob* __restrict__ j
       wave_gemv<T, S, 1, NR>(t, c0, vw);
     return;
   }
-  const PairJob t = jobs[blockIdx.x];
+  const PairJob t = read_job(jobs, blockIdx.x);
   const S* B = static_cast<const S*>(t.B);
   const T* vb = static_cast<const T*>(t.v) + (long long)c0 * t.ldv;
   T* ob = static_cast<T*>(t.out) + (long long)c0 * t.ldo;
@@ -734,7 +742,7 @@ __device__ inline void lat_gemv(const S* __restrict__ B, long long ld, int n, in
 template <class T, class S, int NR>
 __global__ void __launch_bounds__(256) k_pair_gemv_lat(const PairJob* __restrict__ jobs, int c0) {
   __shared__ __align__(16) T xs[lat_elems<T>()];
-  const PairJob t = jobs[blockIdx.x];
+  const PairJob t = read_job(jobs, blockIdx.x);
   const S* B = static_cast<const S*>(t.B);
   const T* vb = static_cast<const T*>(t.v) + (long long)c0 * t.ldv;
   T* ob = static_cast<T*>(t.out) + (long long)c0 * t.ldo;

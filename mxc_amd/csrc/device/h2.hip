@@ -36,7 +36,9 @@ __global__ void __launch_bounds__(256) k_copy2d(const Copy2d<T>* __restrict__ ta
                                                 int ntasks) {
   const long long blk = blockIdx.x;
   const int t = find_task(prefix, ntasks, blk);
-  const Copy2d<T> c = tasks[t];
+  Copy2d<T> c = tasks[t];
+  c.src = in_global(c.src);
+  c.dst = in_global(c.dst);
   const long long e = (blk - prefix[t]) * 256 + threadIdx.x;
   if (e >= (long long)c.m * c.n) return;
   const int i = (int)(e % c.m), j = (int)(e / c.m);
@@ -82,7 +84,14 @@ struct PostTask {
 // share them; the first also permutes the skeleton indices.
 constexpr int POST_BLOCKS = 8;
 __global__ void __launch_bounds__(256) k_post(const PostTask* __restrict__ tasks) {
-  const PostTask t = tasks[blockIdx.x];
+  PostTask t = in_constant(tasks)[blockIdx.x];
+  t.perm = in_global(t.perm);
+  t.Q = in_global(t.Q);
+  t.R = in_global(t.R);
+  t.S = in_global(t.S);
+  t.Stmp = in_global(t.Stmp);
+  t.T = in_global(t.T);
+  t.W = in_global(t.W);
   const int M = t.M, r = t.r;
   const int first = blockIdx.y * 256 + threadIdx.x, step = gridDim.y * 256;
   if (t.mode == 1) {

@@ -47,7 +47,11 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) k_
   __shared__ __align__(16) double candval[2][NW][GJ_NB];
   __shared__ int rowof[NT], stepof[NT];  // pivot row of a step, step of a pivot row (-1: none yet)
   __shared__ double lg[NW];
-  const LuTask<T> task = tasks[blockIdx.x];
+  LuTask<T> task = in_constant(tasks)[blockIdx.x];
+  task.A = in_global(task.A);
+  task.inv = in_global(task.inv);
+  task.work = in_global(task.work);
+  task.info = in_global(task.info);
   const int n = task.n;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lk = lane >> 4;

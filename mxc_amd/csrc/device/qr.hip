@@ -23,6 +23,36 @@
 namespace mxg {
 namespace {
 
+// This workgroup's task, its pointers known to be global ones.
+__device__ inline QrTask read_task(const QrTask* __restrict__ tasks) {
+  QrTask t = in_constant(tasks)[blockIdx.x];
+  t.A = in_global(t.A);
+  t.tau = in_global(t.tau);
+  return t;
+}
+__device__ inline CpqrTask read_task(const CpqrTask* __restrict__ tasks) {
+  CpqrTask t = in_constant(tasks)[blockIdx.x];
+  t.A = in_global(t.A);
+  t.perm = in_global(t.perm);
+  t.rank_out = in_global(t.rank_out);
+  t.work = in_global(t.work);
+  return t;
+}
+__device__ inline FormQTask read_task(const FormQTask* __restrict__ tasks) {
+  FormQTask t = in_constant(tasks)[blockIdx.x];
+  t.P = in_global(t.P);
+  t.tau = in_global(t.tau);
+  t.Q = in_global(t.Q);
+  t.R = in_global(t.R);
+  return t;
+}
+__device__ inline TrTask read_task(const TrTask* __restrict__ tasks) {
+  TrTask t = in_constant(tasks)[blockIdx.x];
+  t.R0 = in_global(t.R0);
+  t.X = in_global(t.X);
+  return t;
+}
+
 // Rows a lane holds for n rows: the smallest of the compiled counts that fits.
 constexpr int ROW_STEPS[] = {1, 2, 3, 4, 5, 6, 8, 12, 16};
 inline int row_steps(int n) {
@@ -142,7 +172,7 @@ __device__ inline void apply_reflector(const double* x, int len, double tau, dou
 __global__ void __launch_bounds__(256) k_qr(const QrTask* __restrict__ tasks) {
   __shared__ Red red;
   __shared__ double sh_tau;
-  const QrTask t = tasks[blockIdx.x];
+  const QrTask t = read_task(tasks);
   const int size = min(t.m, t.n);
   for (int k = 0; k < size; k++) {
     double* col = t.A + k + (long long)k * t.lda;
@@ -189,7 +219,7 @@ __global__ void __launch_bounds__(512) k_qr_reg(const QrTask* __restrict__ tasks
   constexpr int G = C < 8 ? 4 : 8;
   __shared__ double vs[2][64 * R];
   __shared__ double taus[2];
-  const QrTask t = tasks[blockIdx.x];
+  const QrTask t = read_task(tasks);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int size = min(t.m, t.n);
   double a[C][R];
@@ -268,7 +298,7 @@ __global__ void __launch_bounds__(512) k_qr_reg(const QrTask* __restrict__ tasks
 __global__ void __launch_bounds__(256) k_cpqr(const CpqrTask* __restrict__ tasks) {
   __shared__ Red red;
   __shared__ double sh_tau, sh_maxpivot;
-  const CpqrTask t = tasks[blockIdx.x];
+  const CpqrTask t = read_task(tasks);
   const int K = t.K, M = t.M, size = min(K, M);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   double* upd = t.work;
@@ -399,7 +429,7 @@ __global__ void __launch_bounds__(512) k_cpqr_blocked(const CpqrTask* __restrict
   int* flagged = reinterpret_cast<int*>(aux + nb);
   __shared__ int nflag, nrank;
   __shared__ double sh_tau, sh_beta;
-  const CpqrTask t = tasks[blockIdx.x];
+  const CpqrTask t = read_task(tasks);
   const int K = t.K, M = t.M, size = min(K, M);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   double* A = t.A;
@@ -665,7 +695,7 @@ __global__ void __launch_bounds__(512) k_cpqr_blocked(const CpqrTask* __restrict
 }
 
 __global__ void __launch_bounds__(256) k_formq(const FormQTask* __restrict__ tasks) {
-  const FormQTask t = tasks[blockIdx.x];
+  const FormQTask t = read_task(tasks);
   const int M = t.M;
   for (long long e = threadIdx.x; e < (long long)M * M; e += 256) {
     const int i = (int)(e % M), j = (int)(e / M);
@@ -687,7 +717,7 @@ __global__ void __launch_bounds__(256) k_formq(const FormQTask* __restrict__ tas
 template <int R>
 __global__ void __launch_bounds__(256) k_formq_reg(const FormQTask* __restrict__ tasks) {
   constexpr int G = R <= 8 ? 8 : 4;
-  const FormQTask t = tasks[blockIdx.x];
+  const FormQTask t = read_task(tasks);
   const int M = t.M;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c0 = (blockIdx.y * 4 + wave) * G;
@@ -744,7 +774,7 @@ __global__ void __launch_bounds__(256) k_formq_reg(const FormQTask* __restrict__
 }
 
 __global__ void __launch_bounds__(256) k_trsolve(const TrTask* __restrict__ tasks) {
-  const TrTask t = tasks[blockIdx.x];
+  const TrTask t = read_task(tasks);
   const int r = t.r;
   for (int c = threadIdx.x; c < t.n; c += 256) {
     double* x = t.X + (long long)c * r;
@@ -764,7 +794,7 @@ __global__ void __launch_bounds__(256) k_trsolve(const TrTask* __restrict__ task
 template <int R>
 __global__ void __launch_bounds__(256) k_trsolve_reg(const TrTask* __restrict__ tasks) {
   constexpr int G = 4;
-  const TrTask t = tasks[blockIdx.x];
+  const TrTask t = read_task(tasks);
   const int r = t.r;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c0 = (blockIdx.y * 4 + wave) * G;

@@ -117,7 +117,10 @@ __global__ void __launch_bounds__(512) k_sketch(const SketchTask* __restrict__ t
   __shared__ double Xr[2][KT][3];
   __shared__ double wmax[6][8];  // per wave
   __shared__ int widx[8];
-  const SketchTask tk = tasks[blockIdx.x];
+  SketchTask tk = in_constant(tasks)[blockIdx.x];
+  tk.rows = in_global(tk.rows);
+  tk.cols = in_global(tk.cols);
+  tk.out = in_global(tk.out);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lk = lane >> 4;
   const double inf = __builtin_inf();
@@ -362,7 +365,9 @@ __global__ void __launch_bounds__(256) k_sum_slices(const SliceSum* __restrict__
                                                     int ntasks) {
   const long long blk = blockIdx.x;
   const int t = find_task(prefix, ntasks, blk);
-  const SliceSum tk = tasks[t];
+  SliceSum tk = tasks[t];
+  tk.src = in_global(tk.src);
+  tk.dst = in_global(tk.dst);
   const long long e = (blk - prefix[t]) * 256 + threadIdx.x;
   if (e >= tk.len) return;
   double s = 0.;

@@ -67,12 +67,12 @@ __global__ void __launch_bounds__(256) k_sym_gemv(const SymJob* __restrict__ job
   __shared__ __align__(16) T xs[RC * 16];   // x_i of the chunk, [r][16], zero past NR and past the rows
   __shared__ __align__(16) T xp[SP * NR];   // x_j of the panel, [c][k]
   __shared__ __align__(16) T tr[2 * 64 * 4];  // transposed partial sums of the lower half of the rows
-  const SymJob job = jobs[blockIdx.x];
-  const T* __restrict__ B = static_cast<const T*>(job.B);
-  const T* __restrict__ xi = static_cast<const T*>(job.xi) + (long long)c0 * job.ldv;
-  const T* __restrict__ xj = static_cast<const T*>(job.xj) + (long long)c0 * job.ldv;
-  T* out1 = static_cast<T*>(job.out1) + (long long)c0 * job.ldo;
-  T* out2 = job.out2 ? static_cast<T*>(job.out2) + (long long)c0 * job.ldo : nullptr;
+  const SymJob job = in_constant(jobs)[blockIdx.x];
+  const T* __restrict__ B = in_global(static_cast<const T*>(job.B));
+  const T* __restrict__ xi = in_global(static_cast<const T*>(job.xi)) + (long long)c0 * job.ldv;
+  const T* __restrict__ xj = in_global(static_cast<const T*>(job.xj)) + (long long)c0 * job.ldv;
+  T* out1 = in_global(static_cast<T*>(job.out1)) + (long long)c0 * job.ldo;
+  T* out2 = job.out2 ? in_global(static_cast<T*>(job.out2)) + (long long)c0 * job.ldo : nullptr;
   const int n = job.n, m = job.m, ld = job.ld;
   const long long ldv = job.ldv, ldo = job.ldo;
   const int t = threadIdx.x, lane = t & 63, wave = wave_index();
