@@ -451,9 +451,9 @@ void gemm_batched(const std::vector<GemmTask<T>>& tasks, const std::vector<GemmS
   const GemmSeg<T>* ps;
   const GemmTile* pp;
   if (st) {
-    pt = st->put(tasks, s);
-    ps = st->put(segs, s);
-    pp = st->put(tiles, s);
+    pt = st->put(tasks);
+    ps = st->put(segs);
+    pp = st->put(tiles);
   } else {
     dt.upload(tasks, s);
     ds.upload(segs, s);
@@ -463,10 +463,13 @@ void gemm_batched(const std::vector<GemmTask<T>>& tasks, const std::vector<GemmS
     pp = dp.p;
   }
   const dim3 grid((unsigned)total);
-  if constexpr (std::is_same<T, float>::value)
-    if (bf16) hipLaunchKernelGGL(k_bgemm_bf16, grid, dim3(256), 0, s, pt, ps, pp);
-  if (!bf16) {
-    auto go = [&](auto k) { hipLaunchKernelGGL(k, grid, dim3(256), 0, s, pt, ps, pp); };
+  auto launch = [=] {
+    auto go = [&](auto k) {
+      hipLaunchKernelGGL(k, grid, dim3(256), 0, s, pt, ps, pp);
+      MXG_HIP(hipGetLastError());
+    };
+    if constexpr (std::is_same<T, float>::value)
+      if (bf16) return go(k_bgemm_bf16);
     // slabs of 32 rows where a short FP32 tile's products would not cover its
     // loads (the FP32 sums over segments with 1 and 2 blocks: 25.0 and 28.1 us
     // against 29.0 and 33.1 with 16); in FP64 they gain nothing
@@ -476,9 +479,13 @@ void gemm_batched(const std::vector<GemmTask<T>>& tasks, const std::vector<GemmS
     else if (cap == 4) go(k_bgemm<T, 4, 1, unsigned>);
     else if (cap == 2) go(k_bgemm<T, 2, KH, unsigned>);
     else go(k_bgemm<T, 1, KH, unsigned>);
+  };
+  if (st) {
+    st->later(launch);
+  } else {
+    launch();
+    MXG_HIP(hipStreamSynchronize(s));  // descriptor arrays are freed on return
   }
-  MXG_HIP(hipGetLastError());
-  if (!st) MXG_HIP(hipStreamSynchronize(s));  // descriptor arrays are freed on return
 }
 
 template void gemm_batched<double>(const std::vector<GemmTask<double>>&, const std::vector<GemmSeg<double>>&, hipStream_t,

@@ -173,17 +173,26 @@ void copy2d_run(const std::vector<Copy2d<T>>& all, hipStream_t s, Stage* st) {
   const Copy2d<T>* pt;
   const long long* pp;
   if (st) {
-    pt = st->put(tasks, s);
-    pp = st->put(prefix, s);
+    pt = st->put(tasks);
+    pp = st->put(prefix);
   } else {
     dt.upload(tasks, s);
     dp.upload(prefix, s);
     pt = dt.p;
     pp = dp.p;
   }
-  hipLaunchKernelGGL(k_copy2d<T>, dim3((unsigned)prefix.back()), dim3(256), 0, s, pt, pp, (int)tasks.size());
-  MXG_HIP(hipGetLastError());
-  if (!st) MXG_HIP(hipStreamSynchronize(s));
+  const unsigned grid = (unsigned)prefix.back();
+  const int n = (int)tasks.size();
+  auto launch = [=] {
+    hipLaunchKernelGGL(k_copy2d<T>, dim3(grid), dim3(256), 0, s, pt, pp, n);
+    MXG_HIP(hipGetLastError());
+  };
+  if (st) {
+    st->later(launch);
+  } else {
+    launch();
+    MXG_HIP(hipStreamSynchronize(s));
+  }
 }
 
 template void copy2d_run<double>(const std::vector<Copy2d<double>>&, hipStream_t, Stage*);

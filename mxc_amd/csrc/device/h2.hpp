@@ -190,7 +190,7 @@ struct Copy2d {
   int m, n, lds, ldd;
   int trans, pad;
 };
-// every copy of the list in one launch (staged as gemm_batched's)
+// every copy of the list in one launch (staged like gemm_batched's)
 template <class T>
 void copy2d_run(const std::vector<Copy2d<T>>& tasks, hipStream_t s, Stage* st = nullptr);
 // launch helpers used by ulv.hip / gmres.hip

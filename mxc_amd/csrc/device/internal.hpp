@@ -41,8 +41,8 @@ struct GemmTask {
 };
 // bf16: FP32 tasks whose inputs are rounded to bfloat16 and multiplied on the
 // bfloat16 matrix cores with FP32 accumulation. With a stage, the descriptor
-// arrays are staged there and the call returns without waiting for the
-// launch; without one it waits, and the caller may free what it passed.
+// arrays and the launch go there, until its flush; without one the call
+// launches and waits, and the caller may free what it passed.
 template <class T>
 void gemm_batched(const std::vector<GemmTask<T>>& tasks, const std::vector<GemmSeg<T>>& segs, hipStream_t s,
                   bool bf16 = false, Stage* st = nullptr);

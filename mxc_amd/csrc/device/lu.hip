@@ -188,14 +188,22 @@ void launch_gj(const std::vector<LuTask<T>>& tasks, hipStream_t s, Stage* st) {
   DevBuf<LuTask<T>> dt;
   const LuTask<T>* pt;
   if (st) {
-    pt = st->put(tasks, s);
+    pt = st->put(tasks);
   } else {
     dt.upload(tasks, s);
     pt = dt.p;
   }
-  hipLaunchKernelGGL((k_gj_inverse<T, NT>), dim3((unsigned)tasks.size()), dim3(NT), lds, s, pt, ldw);
-  MXG_HIP(hipGetLastError());
-  if (!st) MXG_HIP(hipStreamSynchronize(s));
+  const unsigned n = (unsigned)tasks.size();
+  auto launch = [=] {
+    hipLaunchKernelGGL((k_gj_inverse<T, NT>), dim3(n), dim3(NT), lds, s, pt, ldw);
+    MXG_HIP(hipGetLastError());
+  };
+  if (st) {
+    st->later(launch);
+  } else {
+    launch();
+    MXG_HIP(hipStreamSynchronize(s));
+  }
 }
 
 }  // namespace

@@ -111,12 +111,13 @@ struct LevelPlan {
     sch1.bf16 = sch1.bf16 || o.sch1.bf16;
     sch2.bf16 = sch2.bf16 || o.sch2.bf16;
   }
-  // the launches, in order, with their descriptors staged in st: they have
-  // not necessarily run when this returns
+  // the launches, in order, with their descriptors staged in st; those after
+  // the inverses are issued by the caller's flush
   void run(hipStream_t s, Stage* st) const {
     rot1.run(s, st);
     rot2.run(s, st);
     lu_inverse_batched<T>(lu, s, st);
+    st->flush(s);  // the GPU has work while the rest is laid out
     copy2d_run<T>(vtop, s, st);
     vbot.run(s, st);
     rs.run(s, st);
@@ -142,10 +143,11 @@ struct UlvImpl;
 // as when factorized alone (the tasks are the same, only their launch is
 // shared).
 //
-// No launch waits for the previous one on the host: the descriptor arrays go
-// through the context's stage, every level's scratch comes from the
-// context's arena and stays valid until the end, and the plans are kept, so
-// the host plans level t + 1 while the GPU runs level t.
+// No launch waits for the previous one on the host: descriptor arrays and
+// launches go through the context's stage, which is flushed twice a level,
+// every level's scratch comes from the context's arena and stays valid until
+// the end, and the plans are kept, so the host plans level t + 1 while the GPU
+// runs level t.
 template <class T, class S>
 void factorize_batch(const std::vector<UlvImpl<T, S>*>& fs, hipStream_t s) {
   long long depth = 0;
@@ -170,6 +172,7 @@ void factorize_batch(const std::vector<UlvImpl<T, S>*>& fs, hipStream_t s) {
       }
       P.run(s, &st);
       copy2d_run<T>(next, s, &st);
+      st.flush(s);
     }
     for (auto* f : fs) f->finish();
   } catch (...) {
