@@ -19,6 +19,7 @@ struct Pools {
   std::vector<DevPool*> all;
   std::atomic<size_t> kept{0};  // bytes kept by all pools
   std::atomic<size_t> most{0};  // and at most
+  std::atomic<unsigned long long> age{0};
 };
 // never destroyed: buffers may be released while the process ends
 Pools& pools() {
@@ -69,7 +70,8 @@ void* DevPool::take(size_t bytes, size_t* cap) {
     std::lock_guard<std::mutex> lk(mu_);
     auto it = free_.lower_bound(need);
     if (it != free_.end() && it->first <= need + need / 4 + 4096) {
-      void* p = it->second;
+      void* p = it->second.p;
+      by_age_.erase(it->second.age);
       *cap = it->first;
       kept_ -= it->first;
       pools().kept -= it->first;
@@ -87,22 +89,61 @@ void* DevPool::take(size_t bytes, size_t* cap) {
 
 void DevPool::give(void* p, size_t cap) {
   Pools& P = pools();
-  if (P.kept.fetch_add(cap) + cap > P.most.load()) {
-    P.kept -= cap;
+  if (cap > P.most.load()) {
     (void)hipFree(p);
     return;
   }
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    const unsigned long long age = P.age++;
+    by_age_[age] = free_.emplace(cap, Block{p, age});
+    kept_ += cap;
+    P.kept += cap;
+  }
+  if (P.kept.load() <= P.most.load()) return;
+  std::lock_guard<std::mutex> lk(P.mu);
+  while (P.kept.load() > P.most.load()) {
+    DevPool* from = nullptr;
+    unsigned long long first = ~0ull;
+    for (DevPool* q : P.all) {
+      const unsigned long long a = q->oldest();
+      if (a < first) {
+        first = a;
+        from = q;
+      }
+    }
+    if (!from) break;
+    from->evict_oldest();
+  }
+}
+
+unsigned long long DevPool::oldest() {
   std::lock_guard<std::mutex> lk(mu_);
-  kept_ += cap;
-  free_.emplace(cap, p);
+  return by_age_.empty() ? ~0ull : by_age_.begin()->first;
+}
+
+void DevPool::evict_oldest() {
+  void* p = nullptr;
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    if (by_age_.empty()) return;
+    const auto it = by_age_.begin()->second;
+    p = it->second.p;
+    kept_ -= it->first;
+    pools().kept -= it->first;
+    by_age_.erase(by_age_.begin());
+    free_.erase(it);
+  }
+  (void)hipFree(p);
 }
 
 void DevPool::trim() {
   std::lock_guard<std::mutex> lk(mu_);
-  for (auto& b : free_) (void)hipFree(b.second);
+  for (auto& b : free_) (void)hipFree(b.second.p);
   pools().kept -= kept_;
   kept_ = 0;
   free_.clear();
+  by_age_.clear();
 }
 
 size_t DevPool::kept_on(int device) {
