@@ -30,11 +30,17 @@
 #include <vector>
 
 #include "h2.hpp"
+#include "wave.hpp"
 
 namespace mxg {
 namespace {
 
-constexpr int DOT_ROWS = 2048;  // rows per block of the partial sums
+// Rows per block of the partial sums: 256 blocks if there are rows enough, a
+// row a thread at the least. Short vectors are bound by the latency of a
+// thread's rows one after another (2048 rows a block took 13.6 us a launch at
+// N = 8192, 256 take 4.9; 11.5 and 9.0 with eight right-hand sides in FP32 at
+// N = 65536), long ones by the basis's bytes.
+inline int dot_rows(long long n) { return (int)std::min<long long>(2048, std::max<long long>(256, (n / 256 + 255) / 256 * 256)); }
 constexpr int DOT_MAXC = 32;    // columns per pass of k_dots
 
 // Right-hand side q = blockIdx.y: part[(q * nblk + blk) * ncols + c] = sum
@@ -42,14 +48,14 @@ constexpr int DOT_MAXC = 32;    // columns per pass of k_dots
 template <class B>
 __global__ void __launch_bounds__(256) k_dots(const B* __restrict__ V, int ncols, long long ldv, long long ldq,
                                               long long n, const double* __restrict__ w, long long ldw,
-                                              double* __restrict__ part) {
+                                              double* __restrict__ part, int rows) {
   __shared__ double red[4][DOT_MAXC];
   const int q = blockIdx.y;
   const B* Vq = V + (long long)q * ldq;
   const double* wq = w + (long long)q * ldw;
   double* pq = part + ((long long)q * gridDim.x + blockIdx.x) * ncols;
-  const long long r0 = (long long)blockIdx.x * DOT_ROWS;
-  const long long r1 = min(r0 + DOT_ROWS, n);
+  const long long r0 = (long long)blockIdx.x * rows;
+  const long long r1 = min(r0 + rows, n);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int c0 = 0; c0 < ncols; c0 += DOT_MAXC) {
     const int nc = min(DOT_MAXC, ncols - c0);
@@ -65,7 +71,7 @@ __global__ void __launch_bounds__(256) k_dots(const B* __restrict__ V, int ncols
 #pragma unroll
     for (int c = 0; c < DOT_MAXC; c++) {
       if (c < nc) {
-        const double t = wave_sum(s[c]);
+        const double t = wave_total(s[c]);
         if (lane == 0) red[wave][c] = t;
       }
     }
@@ -87,7 +93,7 @@ __global__ void __launch_bounds__(256) k_sum_parts(const double* __restrict__ pa
   const double* pq = part + (long long)q * nblk * ncols;
   double s = 0.;
   for (int b = lane; b < nblk; b += 64) s += pq[(long long)b * ncols + c];
-  s = wave_sum(s);
+  s = wave_total(s);
   if (lane == 0) out[(long long)q * ldo + c] = s;
 }
 
@@ -165,7 +171,7 @@ struct Gmres {
 
   Gmres(mxg_h2_s* a, mxg_ulv_t mm, int restart, int nrhs, bool basis32)
       : A(a), M(mm), n(a->n), m(restart), nr(nrhs), s(a->ctx->stream), f32(basis32) {
-    nblk = (int)ceil_div(n, DOT_ROWS);
+    nblk = (int)ceil_div(n, dot_rows(n));
     ldq = n * (long long)(m + 1);
     ldh = 2 * (m + 1) + 1;
     auto& g = a->ctx->gmres;
@@ -213,7 +219,8 @@ struct Gmres {
   // out_q[0..ncols) = V_q[:, :ncols]^T w_q on the device (out_q = out + q ldh)
   template <class B>
   void dots_dev(const B* Vp, int ncols, long long ldvq, const double* wp, long long ldw, double* out) {
-    hipLaunchKernelGGL(k_dots<B>, dim3(nblk, nr), dim3(256), 0, s, Vp, ncols, n, ldvq, n, wp, ldw, part.p);
+    hipLaunchKernelGGL(k_dots<B>, dim3(nblk, nr), dim3(256), 0, s, Vp, ncols, n, ldvq, n, wp, ldw, part.p,
+                       dot_rows(n));
     MXG_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_sum_parts, dim3((ncols + 3) / 4, nr), dim3(256), 0, s, part.p, nblk, ncols, out, ldh);
     MXG_HIP(hipGetLastError());
@@ -323,63 +330,76 @@ __global__ void k_arnoldi_step(int i, int m, int cgs2, int nr, const double* __r
 // Reference mode: Householder QR of H_q (its copy in W) and of beta e_1, then
 // back substitution, as the reference's H.householderQr().solve(s)
 // (solver.cpp:187-191).
-__global__ void k_cycle_lsq(int m, int cgs2, int nr, const double* __restrict__ H, const double* __restrict__ gv,
-                            const double* __restrict__ beta, const int* __restrict__ kq, const int* __restrict__ active,
-                            double* __restrict__ W, double* __restrict__ y, int* __restrict__ kd) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nr) return;
+// One wave per right-hand side; its first lane does the work, a chain of
+// dependent operations on a few hundred entries, in LDS where they fit (LSQ_LDS
+// bytes; reading each from memory took 132 us for restart 10, now 53).
+constexpr size_t LSQ_LDS = 65536;
+inline size_t lsq_lds(int m) {
+  const size_t need = ((size_t)(m + 1) * (m + 1) + m + 1) * sizeof(double);
+  return need <= LSQ_LDS ? need : 0;
+}
+__global__ void __launch_bounds__(64) k_cycle_lsq(int m, int cgs2, const double* __restrict__ H, const double* __restrict__ gv,
+                                                  const double* __restrict__ beta, const int* __restrict__ kq,
+                                                  const int* __restrict__ active, double* __restrict__ W,
+                                                  double* __restrict__ y, int* __restrict__ kd, int in_lds) {
+  extern __shared__ double sm[];
+  const int q = blockIdx.x, lane = threadIdx.x;
   const int ld = m + 1;
   double* yq = y + (long long)q * ld;
-  for (int t = 0; t <= m; t++) yq[t] = 0.;
   const int k = active[q] ? kq[q] : 0;
-  kd[q] = k;
+  for (int t = lane; t <= m; t += 64) yq[t] = 0.;
+  if (lane == 0) kd[q] = k;
   if (k == 0) return;
   const double* Hq = H + (long long)q * ld * m;
-  if (cgs2) {
-    const double* g = gv + (long long)q * ld;
-    for (int i2 = k - 1; i2 >= 0; i2--) {
-      double v = g[i2];
-      for (int j = i2 + 1; j < k; j++) v -= Hq[i2 + (long long)j * ld] * yq[j];
-      yq[i2] = v / Hq[i2 + (long long)i2 * ld];
+  // H_q's copy A, then the right-hand side in column m; the solution z
+  auto solve = [&](double* A, double* z) {
+    for (int e = lane; e < (k + 1) * k; e += 64) {
+      const int r = e % (k + 1), c = e / (k + 1);
+      A[r + c * ld] = Hq[r + (long long)c * ld];
     }
-    return;
-  }
-  double* A = W + (long long)q * ld * (m + 1);  // H_q copy, then the right-hand side in column m
-  for (int c = 0; c < k; c++)
-    for (int r = 0; r <= k; r++) A[r + (long long)c * ld] = Hq[r + (long long)c * ld];
-  double* sv = A + (long long)m * ld;
-  for (int r = 0; r <= k; r++) sv[r] = r == 0 ? beta[q] : 0.;
-  const int rows = k + 1;
-  for (int c = 0; c < k; c++) {
-    double* x = A + c + (long long)c * ld;
-    const int len = rows - c;
-    double tail = 0.;
-    for (int i = 1; i < len; i++) tail += x[i] * x[i];
-    double tau = 0., bet = x[0];
-    if (tail > 2.2250738585072014e-308) {
-      bet = sqrt(x[0] * x[0] + tail);
-      if (x[0] >= 0.) bet = -bet;
-      const double sc = 1. / (x[0] - bet);
-      for (int i = 1; i < len; i++) x[i] *= sc;
-      tau = (bet - x[0]) / bet;
-    } else {
-      for (int i = 1; i < len; i++) x[i] = 0.;
+    double* sv = A + m * ld;
+    for (int r = lane; r <= k; r += 64) sv[r] = cgs2 ? gv[(long long)q * ld + r] : r == 0 ? beta[q] : 0.;
+    __syncthreads();
+    if (lane == 0) {
+      const int rows = k + 1;
+      for (int c = 0; c < k && !cgs2; c++) {
+        double* x = A + c + c * ld;
+        const int len = rows - c;
+        double tail = 0.;
+        for (int i = 1; i < len; i++) tail += x[i] * x[i];
+        double tau = 0., bet = x[0];
+        if (tail > 2.2250738585072014e-308) {
+          bet = sqrt(x[0] * x[0] + tail);
+          if (x[0] >= 0.) bet = -bet;
+          const double sc = 1. / (x[0] - bet);
+          for (int i = 1; i < len; i++) x[i] *= sc;
+          tau = (bet - x[0]) / bet;
+        } else {
+          for (int i = 1; i < len; i++) x[i] = 0.;
+        }
+        x[0] = bet;
+        for (int j = c + 1; j <= k; j++) {
+          double* colj = (j < k) ? A + c + j * ld : sv + c;
+          double wv = colj[0];
+          for (int i = 1; i < len; i++) wv += x[i] * colj[i];
+          wv *= tau;
+          colj[0] -= wv;
+          for (int i = 1; i < len; i++) colj[i] -= wv * x[i];
+        }
+      }
+      for (int i = k - 1; i >= 0; i--) {
+        double v = sv[i];
+        for (int j = i + 1; j < k; j++) v -= A[i + j * ld] * z[j];
+        z[i] = v / A[i + i * ld];
+      }
     }
-    x[0] = bet;
-    for (int j = c + 1; j <= k; j++) {
-      double* colj = (j < k) ? A + c + (long long)j * ld : sv + c;
-      double wv = colj[0];
-      for (int i = 1; i < len; i++) wv += x[i] * colj[i];
-      wv *= tau;
-      colj[0] -= wv;
-      for (int i = 1; i < len; i++) colj[i] -= wv * x[i];
-    }
-  }
-  for (int i = k - 1; i >= 0; i--) {
-    double v = sv[i];
-    for (int j = i + 1; j < k; j++) v -= A[i + (long long)j * ld] * yq[j];
-    yq[i] = v / A[i + (long long)i * ld];
-  }
+    __syncthreads();
+    for (int t = lane; t < k; t += 64) yq[t] = z[t];
+  };
+  if (in_lds)
+    solve(sm, sm + ld * ld);
+  else
+    solve(W + (long long)q * ld * (m + 1), yq);
 }
 
 // One HIP graph of an inner step's launches (operator and preconditioner),
@@ -551,8 +571,8 @@ void gmres_batch(mxg_h2_s* A, mxg_ulv_t M, const mxg_gmres_opts_t* o, int nr, co
       if (!open) break;
     }
     // least squares per right-hand side, then x_q += V_q y_q
-    hipLaunchKernelGGL(k_cycle_lsq, small, lanes, 0, g.s, m, ref ? 0 : 1, nr, dH, dgv, dbeta, dk, dactive, ws.W.p, g.yd.p,
-                       g.kd.p);
+    hipLaunchKernelGGL(k_cycle_lsq, dim3(nr), dim3(64), lsq_lds(m), g.s, m, ref ? 0 : 1, dH, dgv, dbeta, dk, dactive,
+                       ws.W.p, g.yd.p, g.kd.p, lsq_lds(m) ? 1 : 0);
     MXG_HIP(hipGetLastError());
     g.basis_add(d_x, ldx);
     // true residual of every right-hand side
