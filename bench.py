@@ -296,7 +296,7 @@ def main():
         },
         "construction": {
             "operator_s": round(t_op, 2),
-            "sketch": {"kernel": "k_sketch (FP64 MFMA) + k_sum_slices", "launches": sketch["launches"],
+            "sketch": {"kernel": "k_sketch (fixed point on the 8-bit integer matrix cores) + k_sum_slices", "launches": sketch["launches"],
                        "s": round(sketch["ms"] * 1e-3, 3), "algorithmic_flops": sketch["work"],
                        "tflops": round(sketch["work"] / (sketch["ms"] * 1e-3) / 1e12, 2) if sketch["ms"] else None,
                        "frac_of_fp64_mfma_peak": round(sketch["work"] / (sketch["ms"] * 1e-3) / 1e12 / 78.6, 3)
