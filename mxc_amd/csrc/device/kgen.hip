@@ -67,24 +67,38 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
   const long long j0 = (long long)blockIdx.y * DM_CHUNK, j1 = min(j0 + DM_CHUNK, n);
   double p[4][3];
   d4_t acc[4];
+  __shared__ int far;  // some coordinate is beyond the kernel's reach
+  if (tid == 0) far = 0;
+  bool beyond = false;
 #pragma unroll
   for (int r = 0; r < 4; r++) {
     const long long i = min(row0 + base + 16 * r + lr, n - 1);
 #pragma unroll
-    for (int d = 0; d < 3; d++) p[r][d] = bodies[3 * i + d];
+    for (int d = 0; d < 3; d++) {
+      p[r][d] = bodies[3 * i + d];
+      beyond = beyond || !(fabs(p[r][d]) <= ke.reach);
+    }
     acc[r] = d4_t{0., 0., 0., 0.};
   }
-  for (long long jt = j0; jt < j1; jt += 256) {
+  bool wide = false;
+  for (long long jt = j0; jt < j1 && !wide; jt += 256) {
     const int cnt = (int)min((long long)256, j1 - jt);
     __syncthreads();
     {  // columns past the chunk repeat its last one, with zero right-hand sides
       const long long j = min(jt + tid, j1 - 1);
 #pragma unroll
-      for (int d = 0; d < 3; d++) sp[3 * tid + d] = bodies[3 * j + d];
+      for (int d = 0; d < 3; d++) {
+        const double x = bodies[3 * j + d];
+        sp[3 * tid + d] = x;
+        beyond = beyond || !(fabs(x) <= ke.reach);
+      }
+      if (beyond) far = 1;
 #pragma unroll
       for (int q = 0; q < NR; q++) sx[tid * NR + q] = tid < cnt ? x[j + q * ldx] : 0.;
     }
     __syncthreads();
+    wide = __builtin_amdgcn_readfirstlane(far);
+    if (wide) break;
     for (int c = 0; c < cnt; c += 4) {
       const double* s = sp + 3 * (c + lk);
       const double xb = lr < NR ? sx[(c + lk) * NR + (lr < NR ? lr : 0)] : 0.;
@@ -106,6 +120,23 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
 #pragma unroll
       for (int r = 0; r < 4; r++) acc[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(v[r], xb, acc[r], 0, 0, 0);
     }
+  }
+  if (wide) {
+    // distances that kernel_scaled may not be for: the chunk once more, a row per
+    // thread
+    const long long li = (long long)blockIdx.x * DM_ROWS + tid, i = min(row0 + li, n - 1);
+    const double x0 = bodies[3 * i], x1 = bodies[3 * i + 1], x2 = bodies[3 * i + 2];
+    double sum[NR] = {};
+    for (long long j = j0; j < j1; j++) {
+      const double dx = x0 - bodies[3 * j], dy = x1 - bodies[3 * j + 1], dz = x2 - bodies[3 * j + 2];
+      const double v = kernel_any<KID>(dx * dx + dy * dy + dz * dz, ke);
+#pragma unroll
+      for (int q = 0; q < NR; q++) sum[q] += v * x[j + q * ldx];
+    }
+    if (li < rows && row0 + li < n)
+#pragma unroll
+      for (int q = 0; q < NR; q++) part[((long long)blockIdx.y * NR + q) * ldp + li] = sum[q];
+    return;
   }
   // entry q of lane l: row l / 16 + 4 q of the block, right-hand side l mod 16
   if (lr < NR)
