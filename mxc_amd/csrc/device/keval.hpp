@@ -36,7 +36,7 @@ struct EvalArgs {
 inline EvalArgs eval_args(mxg_kernel_t k) {
   // the product's rounding error and log2(e)'s own tail make the second part
   const double L2E = 1.4426950408889634, L2E_TAIL = 2.0355273740931033e-17, ch = -k.alpha * L2E;
-  double far2 = 0.25 * DBL_MAX;
+  double far2 = DBL_MAX;
   if (k.id == MXG_KERNEL_YUKAWA || k.id == MXG_KERNEL_GAUSSIAN) {
     // an exponent of at most 2^30 in magnitude
     const double d = 1073741824.0 / std::fabs(ch), d2 = k.id == MXG_KERNEL_YUKAWA ? d * d : d;

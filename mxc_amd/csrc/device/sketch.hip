@@ -107,7 +107,7 @@ __device__ inline void bytes_of(unsigned a, unsigned b, unsigned c, unsigned d, 
 // 16 x 16; KT far rows per step.
 template <int KID, int WR, int RW, int CT, int KT>
 __global__ void __launch_bounds__(512) k_sketch(const SketchTask* __restrict__ tasks, const double* __restrict__ bodies,
-                                                double alpha, EvalArgs ke, const u4* __restrict__ signs, int nu) {
+                                                EvalArgs ke, const u4* __restrict__ signs, int nu) {
   constexpr int WC = 8 / WR, TC = 16 * CT * WC;
   constexpr int E = KT * TC / 512;  // entries a thread evaluates per step: consecutive rows of one column
   constexpr int SUB = 16 / E;       // threads sharing 16 rows of a column
@@ -131,8 +131,9 @@ __global__ void __launch_bounds__(512) k_sketch(const SketchTask* __restrict__ t
   const double x0 = bodies[3 * cb], x1 = bodies[3 * cb + 1], x2 = bodies[3 * cb + 2];
 
   // ---- bound of the entries ----
-  int shift;           // entries are K 2^shift, below 2^60
-  bool zeros = false;  // some pairs coincide
+  int shift;         // entries are K 2^shift, below 2^60
+  bool odd = false;  // some distances are not for kernel_scaled: zero (the diagonal value), or
+                     // beyond ke.far2, where entries are zero if they are finite
   {
     // largest over the workgroup of N values, in every thread
     auto wg_max = [&](auto& v) {
@@ -151,29 +152,33 @@ __global__ void __launch_bounds__(512) k_sketch(const SketchTask* __restrict__ t
         for (int w = 1; w < 8; w++) v[d] = fmax(v[d], wmax[d][w]);
       }
     };
-    // the row nearest to the bounding box of the tile's columns
+    // the row nearest to the bounding box of the tile's columns, and how far any
+    // row can be from a column
     bool nan = !(x0 == x0 && x1 == x1 && x2 == x2);
     double hull[6] = {x0, x1, x2, -x0, -x1, -x2};
     wg_max(hull);
-    double best = inf;
+    double best = inf, most = 0.;
     int at = tk.t0;
 #pragma unroll 4
     for (int t = tk.t0 + tid; t < tk.t0 + SKETCH_ROWS; t += 512) {
       const int tc = min(t, tk.t1 - 1);
       const double* r = bodies + 3 * (long long)tk.rows[tc];
-      double d2 = 0.;
+      double d2 = 0., far2 = 0.;
 #pragma unroll
       for (int d = 0; d < 3; d++) {
-        const double x = r[d], g = fmax(fmax(-hull[3 + d] - x, x - hull[d]), 0.);
+        const double x = r[d], below = -hull[3 + d] - x, above = x - hull[d];
+        const double g = fmax(fmax(below, above), 0.), f = fmin(below, above);
         nan = nan || !(x == x);
         d2 += g * g;
+        far2 += f * f;
       }
       if (d2 < best) { best = d2; at = tc; }
+      most = fmax(most, far2);
     }
     const double wbest = -wave_max(-best);
     const int src = __ffsll((long long)__ballot(best == wbest)) - 1;
     if (lane == src) widx[wave] = at;
-    double lo[1] = {-wbest};
+    double lo[2] = {-wbest, most};
     wg_max(lo);
 #pragma unroll
     for (int w = 0; w < 8; w++)
@@ -185,9 +190,9 @@ __global__ void __launch_bounds__(512) k_sketch(const SketchTask* __restrict__ t
     const double e0 = r[0] - x0, e1 = r[1] - x1, e2 = r[2] - x2;
     double has[1] = {-(e0 * e0 + e1 * e1 + e2 * e2)};
     wg_max(has);
-    double bound = lo2 > 0. ? kernel_eval(KID, ke.diag, alpha, lo2) : inf;
-    const bool falls = KID == MXG_KERNEL_LAPLACE || alpha >= 0.;
-    if (!falls || has[0] == 0. || !(bound <= 64. * kernel_eval(KID, ke.diag, alpha, -has[0]))) {
+    const bool falls = KID == MXG_KERNEL_LAPLACE || ke.ch <= 0., plain = lo2 > 0. && lo[1] <= 0.5 * ke.far2;
+    double bound = plain ? kernel_any<KID>(lo2, ke) : inf;
+    if (!falls || !plain || has[0] == 0. || !(bound <= 64. * kernel_any<KID>(-has[0], ke))) {
       // the extreme distances over all pairs, the rows staged 512 at a time; a
       // coinciding pair has the diagonal value
       double* st = reinterpret_cast<double*>(&Gs[0][0][0][0][0]);
@@ -210,10 +215,11 @@ __global__ void __launch_bounds__(512) k_sketch(const SketchTask* __restrict__ t
         }
       }
       wg_max(ext);
-      bound = fmax(ext[0] > -inf ? kernel_eval(KID, ke.diag, alpha, -ext[0]) : 0.,
-                   ext[1] > 0. ? kernel_eval(KID, ke.diag, alpha, ext[1]) : 0.);
-      zeros = ext[2] > 0.;
-      if (zeros) bound = fmax(bound, fabs(kernel_eval(KID, ke.diag, alpha, 0.)));
+      const double last = ext[1] > 0. ? kernel_any<KID>(ext[1], ke) : 0.;
+      bound = fmax(ext[0] > -inf ? kernel_any<KID>(-ext[0], ke) : 0., last);
+      if (ext[2] > 0.) bound = fmax(bound, fabs(ke.diag));
+      if (!(last < inf)) bound = inf;
+      odd = ext[2] > 0. || !(ext[1] <= ke.far2);
       __syncthreads();  // the staged rows have been read
     }
     if (nan || !(bound < inf)) {  // entries that are not finite make the tile NaN
@@ -247,12 +253,13 @@ __global__ void __launch_bounds__(512) k_sketch(const SketchTask* __restrict__ t
   };
   // the bytes of this thread's entries of step tb into buffer b
   auto store = [&](int tb, int b, double (&v)[E]) {
-    if (zeros) {
+    if (odd) {
 #pragma unroll
       for (int e = 0; e < E; e++) {
         const int tt = 16 * tg + sub * E + e;
-        if (Xr[b][tt][0] == x0 && Xr[b][tt][1] == x1 && Xr[b][tt][2] == x2)
-          v[e] = ldexp(ke.diag, shift - 30);
+        const double dx = Xr[b][tt][0] - x0, dy = Xr[b][tt][1] - x1, dz = Xr[b][tt][2] - x2;
+        const double d2 = dx * dx + dy * dy + dz * dz;
+        v[e] = d2 == 0. ? ldexp(ke.diag, shift - 30) : d2 > ke.far2 ? 0. : v[e];
       }
     }
     if (tb + KT > tk.t1) {
@@ -394,11 +401,11 @@ void launch_sketch(int shape, unsigned grid, const SketchTask* tasks, const doub
   const dim3 g(grid), blk(512);
   const EvalArgs ke = eval_args(k);
   switch (shape) {
-    case 0: hipLaunchKernelGGL((k_sketch<KID, 4, 1, 2, 64>), g, blk, 0, s, tasks, bodies, k.alpha, ke, signs, nu); break;
-    case 1: hipLaunchKernelGGL((k_sketch<KID, 8, 1, 4, 64>), g, blk, 0, s, tasks, bodies, k.alpha, ke, signs, nu); break;
-    case 2: hipLaunchKernelGGL((k_sketch<KID, 8, 2, 2, 64>), g, blk, 0, s, tasks, bodies, k.alpha, ke, signs, nu); break;
-    case 3: hipLaunchKernelGGL((k_sketch<KID, 8, 3, 2, 64>), g, blk, 0, s, tasks, bodies, k.alpha, ke, signs, nu); break;
-    default: hipLaunchKernelGGL((k_sketch<KID, 8, 4, 1, 128>), g, blk, 0, s, tasks, bodies, k.alpha, ke, signs, nu); break;
+    case 0: hipLaunchKernelGGL((k_sketch<KID, 4, 1, 2, 64>), g, blk, 0, s, tasks, bodies, ke, signs, nu); break;
+    case 1: hipLaunchKernelGGL((k_sketch<KID, 8, 1, 4, 64>), g, blk, 0, s, tasks, bodies, ke, signs, nu); break;
+    case 2: hipLaunchKernelGGL((k_sketch<KID, 8, 2, 2, 64>), g, blk, 0, s, tasks, bodies, ke, signs, nu); break;
+    case 3: hipLaunchKernelGGL((k_sketch<KID, 8, 3, 2, 64>), g, blk, 0, s, tasks, bodies, ke, signs, nu); break;
+    default: hipLaunchKernelGGL((k_sketch<KID, 8, 4, 1, 128>), g, blk, 0, s, tasks, bodies, ke, signs, nu); break;
   }
   MXG_HIP(hipGetLastError());
 }

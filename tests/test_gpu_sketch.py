@@ -1,10 +1,14 @@
 """The far-field sketch (sketch.hip) at the edges of its tiles, slices and
 scaling: ranks and interpolative bases against the oracle's FP64 sketch of the
 same blocks, and the product against the dense one."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import oracle_lib as O
+from mxc_amd import _native as N
+from mxc_amd.device import kernel_desc
 from mxc_amd.solver import H2, Problem
 
 pytestmark = pytest.mark.gpu
@@ -55,3 +59,55 @@ def test_coinciding_points(ctx):
     pts = O.cube_points(1200, 24).reshape(-1, 3)
     pts[300:900] = pts[0]
     check(ctx, pts.reshape(-1), 150, same_bases=False)
+
+
+def first_basis(ctx, pts, M, far, kernel, diag=1e3, alpha=1.0):
+    """Rank and interpolative basis (M x M) of the box of the first M points for an explicit far list."""
+    G, n = N.gpu(), len(pts)
+    i64 = lambda *a: np.array(a, np.int64)  # noqa: E731
+    pts, far = np.ascontiguousarray(pts), np.asarray(far, np.int64)
+    dims, begin, rp, col, none = i64(M, n - M), i64(0, M), i64(0, 2, 4), i64(0, 1, 0, 1), i64(0, 0, 0)
+    off, ranks = i64(0, len(far), len(far)), i64(0, 0)
+    h = C.c_void_p()
+    N.check_gpu(G.mxg_h2_create(ctx.handle, kernel_desc(kernel, diag, alpha), pts.ctypes.data, n, 1, 0, C.byref(h)))
+    N.check_gpu(G.mxg_h2_construct_level(h, 1, 2, *(a.ctypes.data for a in (dims, begin, rp, col, none, none, off, far)),
+                                         1e-2, 0, 0, ranks.ctypes.data))
+    q = np.zeros(G.mxg_h2_level_size(h, 1, N.H2_BASIS))
+    N.check_gpu(G.mxg_h2_download(h, 1, N.H2_BASIS, q.ctypes.data, len(q)))
+    G.mxg_h2_destroy(h)
+    return ranks[0], q[:M * M].reshape(M, M).T
+
+
+def apart(M, rows, seed):
+    """M points in a cube of side 0.2 amid rows outside of a cube of side 0.4, the first row but one in its middle."""
+    p = O.cube_points(M + 2 * rows, seed).reshape(-1, 3)
+    cols, others = 0.4 + 0.2 * p[:M], p[M:]
+    others = others[np.abs(others - 0.5).max(1) > 0.2][:rows]
+    others[1] = [0.5, 0.503, 0.5]
+    return np.concatenate([cols, others])
+
+
+@pytest.mark.parametrize("M", [40, 300])
+@pytest.mark.parametrize("kernel,away", [("laplace", [1e155, 1e160]), ("yukawa", [1e12, 1e155, 1e160]),
+                                         ("gaussian", [1e7, 1e155, 1e160])])
+def test_far_rows_with_zero_entries(ctx, M, kernel, away):
+    """Rows whose squared distance overflows, or whose exponential is zero, add nothing."""
+    pts = apart(M, 700 + len(away), 25)
+    pts[M + 700:] = np.array(away)[:, None] * [1.0, -0.5, 0.25]
+    far = np.arange(M, len(pts))
+    r, q = first_basis(ctx, pts, M, far, kernel)
+    r0, q0 = first_basis(ctx, pts, M, far[:700], kernel)
+    assert 0 < r0 < M and np.isfinite(q0).all()
+    assert r == r0 and np.array_equal(q, q0)
+
+
+@pytest.mark.parametrize("M", [40, 300])
+@pytest.mark.parametrize("kernel", ["laplace", "yukawa", "gaussian"])
+def test_distances_that_underflow(ctx, M, kernel):
+    """A far row at a distance whose square is zero has the diagonal value, as if it coincided."""
+    pts = apart(M, 700, 26) - 0.5
+    pts[3] = pts[M + 5] = 0.0
+    r0, q0 = first_basis(ctx, pts, M, np.arange(M, len(pts)), kernel)
+    pts[M + 5] = [1e-170, 0.0, 0.0]
+    r, q = first_basis(ctx, pts, M, np.arange(M, len(pts)), kernel)
+    assert 0 < r0 < M and r == r0 and np.array_equal(q, q0)
