@@ -117,6 +117,7 @@ __global__ void __launch_bounds__(512) k_sketch(const SketchTask* __restrict__ t
   __shared__ double Xr[2][KT][3];
   __shared__ double wmax[6][8];  // per wave
   __shared__ int widx[8];
+  __shared__ unsigned char bad[TC];  // columns with entries that are not finite
   SketchTask tk = in_constant(tasks)[blockIdx.x];
   tk.rows = in_global(tk.rows);
   tk.cols = in_global(tk.cols);
@@ -134,6 +135,7 @@ __global__ void __launch_bounds__(512) k_sketch(const SketchTask* __restrict__ t
   int shift;         // entries are K 2^shift, below 2^60
   bool odd = false;  // some distances are not for kernel_scaled: zero (the diagonal value), or
                      // beyond ke.far2, where entries are zero if they are finite
+  bool flagged = false;  // bad is in use
   {
     // largest over the workgroup of N values, in every thread
     auto wg_max = [&](auto& v) {
@@ -215,19 +217,30 @@ __global__ void __launch_bounds__(512) k_sketch(const SketchTask* __restrict__ t
         }
       }
       wg_max(ext);
-      const double last = ext[1] > 0. ? kernel_any<KID>(ext[1], ke) : 0.;
-      bound = fmax(ext[0] > -inf ? kernel_any<KID>(-ext[0], ke) : 0., last);
-      if (ext[2] > 0.) bound = fmax(bound, fabs(ke.diag));
-      if (!(last < inf)) bound = inf;
+      bound = ext[2] > 0. ? fabs(ke.diag) : 0.;
+      const double nearest = ext[0] > -inf ? kernel_any<KID>(-ext[0], ke) : 0., farthest = ext[1] > 0. ? kernel_any<KID>(ext[1], ke) : 0.;
+      // not a number, or infinite: at least one of the three is
+      flagged = nan || !(bound < inf && nearest < inf && farthest < inf);
+      bound = fmax(bound, fmax(nearest, farthest));
       odd = ext[2] > 0. || !(ext[1] <= ke.far2);
       __syncthreads();  // the staged rows have been read
     }
-    if (nan || !(bound < inf)) {  // entries that are not finite make the tile NaN
-      for (int e = tid; e < TC * 16 * WR * RW; e += 512) {
-        const int row = tk.i0 + e % (16 * WR * RW), c = tk.j0 + e / (16 * WR * RW);
-        if (row < tk.M && c < tk.M) tk.out[row + (long long)c * tk.M] = __builtin_nan("");
+    flagged = flagged || nan;
+    if (flagged) {
+      // the columns of such entries will be NaN, as their sums are; the others' bound
+      if (tid < TC) bad[tid] = 0;
+      __syncthreads();
+      double big[1] = {0.};
+      for (int t = tk.t0 + tg * SUB + sub; t < tk.t1; t += TG * SUB) {
+        const double* q = bodies + 3 * (long long)tk.rows[t];
+        const double dx = q[0] - x0, dy = q[1] - x1, dz = q[2] - x2;
+        const double v = fabs(kernel_any<KID>(dx * dx + dy * dy + dz * dz, ke));
+        if (v < inf) big[0] = fmax(big[0], v);
+        else bad[col] = 1;
       }
-      return;
+      wg_max(big);
+      bound = big[0];
+      odd = true;
     }
     shift = __builtin_amdgcn_readfirstlane(bound > 0. ? 59 - ilogb(bound) : 0);
   }
@@ -363,7 +376,8 @@ __global__ void __launch_bounds__(512) k_sketch(const SketchTask* __restrict__ t
           hi = hi * 256 + acc[i][j][4 + s][q];
         }
         const double y = ldexp(fma((double)hi, 1073741824.0, (double)lo), -shift);
-        if (row < tk.M && c < tk.M) tk.out[row + (long long)c * tk.M] = y;
+        const bool drop = flagged && bad[(wc * CT + j) * 16 + lr];
+        if (row < tk.M && c < tk.M) tk.out[row + (long long)c * tk.M] = drop ? __builtin_nan("") : y;
       }
 }
 

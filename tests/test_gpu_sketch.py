@@ -111,3 +111,30 @@ def test_distances_that_underflow(ctx, M, kernel):
     pts[M + 5] = [1e-170, 0.0, 0.0]
     r, q = first_basis(ctx, pts, M, np.arange(M, len(pts)), kernel)
     assert 0 < r0 < M and r == r0 and np.array_equal(q, q0)
+
+
+@pytest.mark.parametrize("M", [40, 300])
+@pytest.mark.parametrize("case", ["diagonal", "column", "overflow"])
+def test_columns_that_are_not_finite(ctx, M, case):
+    """Entries that are not finite spoil their own columns, visibly: a diagonal value that is NaN with coinciding
+    points, a column point that is NaN, a kernel that overflows for one pair. The others' bases are as ever."""
+    pts = apart(M, 700, 27)
+    col, diag, kernel, alpha = 3, 1e3, "laplace", 1.0
+    far = np.arange(M, len(pts))
+    if case == "diagonal":
+        pts[M + 9], diag = pts[col], np.nan
+    elif case == "column":
+        pts[col] = np.nan
+    else:
+        kernel, alpha = "gaussian", -200.0  # columns of squares that are still finite
+        pts[M + 10] = [10.0, 0.5, 0.5]
+        far = far[far != M + 10]
+        pts[col] = [9.5, 0.5, 0.5]  # 9 from the other columns' middle: exp(200 81) against every row
+    r, q = first_basis(ctx, pts, M, far, kernel, diag, alpha)
+    assert 0 < r < M
+    rest = np.arange(M) != col
+    assert np.isnan(q[col, :r]).all() and np.isfinite(q[rest]).all()
+    # the same with a column of zeros in its place, or for a kernel without any, of NaN
+    pts[col] = np.nan if case == "overflow" else 1e160
+    r0, q0 = first_basis(ctx, pts, M, far, kernel, 1e3, alpha)
+    assert r == r0 and np.abs(q[rest] - q0[rest]).max() < 1e-9
