@@ -330,6 +330,7 @@ __global__ void __launch_bounds__(256) k_cpqr(const CpqrTask* __restrict__ tasks
     double gv;
     int gi;
     wg_argmax(bv, bi, red, gv, gi);
+    if (gi >= M) gi = k;  // no comparable norm (NaN): the columns in order
     if (nonzero == size && gv * gv < th_helper * (double)(K - k)) nonzero = k;
     if (t.tol > 0. && nonzero < size) break;                      // rank counts i < nonzero only
     if (t.tol > 0. && k > 0 && gv <= t.tol * maxpivot) break;    // every later |R_ii| is below the threshold
@@ -388,7 +389,7 @@ __global__ void __launch_bounds__(256) k_cpqr(const CpqrTask* __restrict__ tasks
       const double th = maxpivot * t.tol;
       const int lim = min(nonzero, done);
       rank = 0;
-      for (int i = 0; i < lim; i++) rank += fabs(t.A[i + (long long)i * t.lda]) > th;
+      for (int i = 0; i < lim; i++) rank += !(fabs(t.A[i + (long long)i * t.lda]) <= th);  // NaN counts
     } else {
       rank = done;
     }
@@ -683,7 +684,7 @@ __global__ void __launch_bounds__(512) k_cpqr_blocked(const CpqrTask* __restrict
     const double th = maxpivot * t.tol;
     const int lim = min(nonzero, done);
     int mine = 0;
-    for (int i = tid; i < lim; i += 512) mine += diag[i] > th;
+    for (int i = tid; i < lim; i += 512) mine += !(diag[i] <= th);  // NaN counts, so that it shows
     if (mine) atomicAdd(&nrank, mine);
     __syncthreads();
   }

@@ -7,6 +7,7 @@ import pytest
 
 import oracle_lib as O
 from mxc_amd.solver import H2, Problem
+from test_gpu_sketch import first_basis
 
 pytestmark = pytest.mark.gpu
 
@@ -67,3 +68,12 @@ def test_rows_reduced_by_householder(ctx, M):
     prob.dense_matvec("laplace", 1e3, 0.0, x, z)
     # interpolation error: the truncated pivots times a modest growth factor
     assert O.rel_err(y.download(), z.download()) < 1e-9 * 4 * M
+
+
+@pytest.mark.parametrize("M", [40, 300, 1100])
+def test_no_comparable_norm(ctx, M):
+    """A far point that is NaN makes every column's norm NaN: the basis shows it (and no column past the last is read)."""
+    pts = O.cube_points(2 * M, 14).reshape(-1, 3)
+    pts[M + M // 2] = np.nan
+    r, q = first_basis(ctx, pts, M, np.arange(M, 2 * M), "laplace")
+    assert r > 0 and np.isnan(q).any()
