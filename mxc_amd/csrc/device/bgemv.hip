@@ -1205,7 +1205,7 @@ template void comb_fwd<double>(const Level&, const long long*, const double*, lo
 template <class T>
 void bwd_gather(const Level& Lv, const long long* d_toff, const T* x, long long ldx, const T* w, long long ldw, const T* t,
                 long long ldt, T* v, long long ldv, int nrhs, hipStream_t s) {
-  if (Lv.nb == 0) return;
+  if (Lv.nb == 0 || Lv.lenX == 0) return;
   hipLaunchKernelGGL(k_bwd_gather<T>, dim3((unsigned)Lv.nb, ceil_div(Lv.maxM * nrhs, 256)), dim3(256), 0, s, Lv.d_dims.p, Lv.d_ranks.p, Lv.d_offX.p,
                      Lv.d_offZ.p, Lv.d_nrp.p, d_toff, x, w, t, v, Strides{ldx, ldw, ldt, ldv}, nrhs);
   MXG_HIP(hipGetLastError());

@@ -7,7 +7,7 @@ import pytest
 
 import oracle_lib as O
 from mxc_amd import _native as N
-from mxc_amd.solver import H2, Problem
+from mxc_amd.solver import H2, HostLevels, Problem
 
 pytestmark = pytest.mark.gpu
 
@@ -73,3 +73,29 @@ def test_more_terms_than_staged(ctx):
     oM = O.Problem(pts, 2).h2(rank=1, orth=True, hss_far=True, theta=1e6)
     oM.factorize()
     assert O.rel_err(dx.download(), oM.precondition(x)) < 1e-8
+
+
+@pytest.mark.parametrize("precision,tol", [(N.MXG_FP64, 1e-12), (N.MXG_FP32, 1e-4), (N.MXG_BF16, 1e-1)])
+def test_levels_of_empty_boxes(ctx, precision, tol):
+    """Leaves of rank 0: the boxes above have no rows. The matrix is its diagonal blocks."""
+    n, leaf = 132, 33
+    prob = Problem(ctx, O.cube_points(n, 43), leaf)
+    assert prob.levels == 2
+    rng = np.random.default_rng(4)
+    blocks = [rng.uniform(-1, 1, (leaf, leaf)) + 8 * np.eye(leaf) for _ in range(4)]
+    alone = [((np.arange(b + 1), np.arange(b)), (np.zeros(b + 1), np.zeros(0))) for b in (1, 2, 4)]
+    levels = [dict(dims=[0] * b, ranks=[0] * b, near=near, far=far) for b, (near, far) in zip((1, 2), alone)]
+    levels.append(dict(dims=[leaf] * 4, ranks=[0] * 4, near=alone[2][0], far=alone[2][1],
+                       A=np.concatenate([b.T.reshape(-1) for b in blocks])))
+    M = HostLevels(prob, levels)
+    assert not M.factorize(precision).any()
+    for nr in (1, 2, 3, 4, 8):
+        x = rng.uniform(-1, 1, (n, nr))
+        ref = np.concatenate([b @ x[leaf * i:leaf * i + leaf] for i, b in enumerate(blocks)])
+        inv = np.concatenate([np.linalg.solve(b, x[leaf * i:leaf * i + leaf]) for i, b in enumerate(blocks)])
+        dx, dy = ctx.array(x), ctx.zeros((n, nr))
+        M.matvec(dx, dy)
+        assert O.rel_err(dy.download().reshape(-1), ref.reshape(-1)) < 1e-13
+        M.precondition(dx)  # blocks of condition about 10: rounding, or storage
+        assert O.rel_err(dx.download().reshape(-1), inv.reshape(-1)) < tol, nr
+    M.close()
