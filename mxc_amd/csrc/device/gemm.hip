@@ -286,7 +286,9 @@ __global__ void __launch_bounds__(256, sizeof(T) == 8 && CAP == 8 ? 3 : 4) k_bge
 // bfloat16 (nearest even) as they are staged, and each 16-deep slab is one
 // v_mfma_f32_16x16x16_bf16 per 16 x 16 accumulator (FP32 accumulation). Lane l
 // supplies A[l % 16][4 (l / 16) + e] and B[4 (l / 16) + e][l % 16], e < 4; the
-// accumulator layout is that of the FP32 instruction.
+// accumulator layout is that of the FP32 instruction. Tiles go to the XCDs in runs,
+// by the table, or (RUNS false) in launch order, each workgroup finding its task in
+// the prefix sums of the tasks' tiles.
 typedef short s4_t __attribute__((ext_vector_type(4)));
 constexpr int BM = 64, BN = 64, BK = 16, PADH = 2;
 
@@ -295,12 +297,22 @@ __device__ inline unsigned short bf16_bits(float x) {
   return (unsigned short)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
 }
 
+template <bool RUNS>
 __global__ void __launch_bounds__(256) k_bgemm_bf16(const GemmTask<float>* __restrict__ tasks,
                                                     const GemmSeg<float>* __restrict__ segs,
-                                                    const GemmTile* __restrict__ tiles) {
+                                                    const GemmTile* __restrict__ tiles,
+                                                    const long long* __restrict__ prefix, int ntasks) {
   __shared__ unsigned short As[BK][BM + PADH];
   __shared__ unsigned short Bs[BK][BN + PADH];
-  const GemmTile tile = my_tile(tiles);
+  GemmTile tile;
+  if constexpr (RUNS) {
+    tile = my_tile(tiles);
+  } else {
+    tile.task = find_task(prefix, ntasks, blockIdx.x);
+    const int local = (int)(blockIdx.x - prefix[tile.task]), tiles_m = (in_constant(tasks)[tile.task].m + BM - 1) / BM;
+    tile.f0 = local % tiles_m * BM;
+    tile.s0 = local / tiles_m * BN;
+  }
   const GemmTask<float> task = in_constant(tasks)[tile.task];
   const int m0 = tile.f0, n0 = tile.s0;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -425,51 +437,75 @@ void gemm_batched(const std::vector<GemmTask<T>>& tasks, const std::vector<GemmS
   // 4, 955 with 2), short ones keep a small launch's chip busy (one tile of 16
   // to 128 rows of 64 Schur sums, K = 2660: 296, 307, 369 and 523 us with 1, 2,
   // 4 and 8 blocks).
-  int cap = bf16 ? 4 : 8;
+  int cap = 8;
   while (!bf16 && cap > 1 && count_tiles(tasks, cap) < 512) cap /= 2;
   // byte offsets of a tile's entries in 32 bits, unless a column stride is 2^21 or more
   bool wide = false;
   for (const GemmSeg<T>& g : segs) wide = wide || std::max(g.lda, g.ldb) >= (1 << 21);
-  if (wide && !bf16) cap = 4;
+  if (wide) cap = 4;
   std::vector<GemmTile> tiles;
-  for (size_t t = 0; t < tasks.size(); t++) {
+  std::vector<long long> prefix;  // of the bfloat16 tasks' tiles, if they go in launch order
+  if (bf16) {
+    prefix.push_back(0);
+    for (const GemmTask<T>& g : tasks)
+      prefix.push_back(prefix.back() +
+                       (g.m > 0 && g.n > 0 ? (long long)((g.m + BM - 1) / BM) * ((g.n + BN - 1) / BN) : 0));
+    MXG_REQUIRE(prefix.back() < (1ll << 31), "gemm grid too large");
+    // The blocks of a factorization share their operands within a run (N = 20000,
+    // rank 100, with bfloat16 Schur products: 7.5 ms, 8.0 in launch order). An XCD
+    // that takes a run of a large block's columns reads all rows of op(A) at once,
+    // beyond its L2: from 64 tiles on in launch order if A is stored as it is used
+    // (4096 x 256 x 4096: 537 us, 580 in runs; 1000 x 1000 x 1000: 182 and 196), from
+    // 1024 on if it is transposed (4096 x 4096 x 1024: 472 and 549; but 256 x 4096 x
+    // 4096: 498 and 447, 1000 x 1000 x 1000: 200 and 181).
+    bool ta = false;
+    for (const GemmSeg<T>& g : segs) ta = ta || g.ta;
+    if (prefix.back() <= (ta ? 1023 : 64) * (long long)tasks.size()) prefix.clear();
+  }
+  const bool runs = prefix.empty();
+  for (size_t t = 0; t < tasks.size() && runs; t++) {
     const GemmTask<T>& g = tasks[t];
     if (g.m <= 0 || g.n <= 0) continue;
-    Tiling c = tiling(g.m, g.n, cap);
-    if (bf16) c = Tiling{(g.m + 63) / 64, (g.n + 63) / 64, 4, 0};
+    const Tiling c = bf16 ? Tiling{(g.m + BM - 1) / BM, (g.n + BN - 1) / BN, 4, 0} : tiling(g.m, g.n, cap);
     MXG_REQUIRE(tiles.size() + c.nf * c.ns < (1ull << 31), "gemm grid too large");
     for (long long y = 0; y < c.ns; y++)
       for (long long x = 0; x < c.nf; x++)
         tiles.push_back(GemmTile{(int)t, (int)(x * 16 * c.mi), (int)(y * 64), (short)c.mi, (short)c.swap});
   }
-  if (tiles.empty()) return;
-  const size_t total = tiles.size();
+  const size_t total = runs ? tiles.size() : (size_t)prefix.back();
+  if (total == 0) return;
   DevBuf<GemmTask<T>> dt;
   DevBuf<GemmSeg<T>> ds;
   DevBuf<GemmTile> dp;
+  DevBuf<long long> dx;
   const GemmTask<T>* pt;
   const GemmSeg<T>* ps;
   const GemmTile* pp;
+  const long long* px;
   if (st) {
     pt = st->put(tasks);
     ps = st->put(segs);
     pp = st->put(tiles);
+    px = st->put(prefix);
   } else {
     dt.upload(tasks, s);
     ds.upload(segs, s);
     dp.upload(tiles, s);
+    dx.upload(prefix, s);
     pt = dt.p;
     ps = ds.p;
     pp = dp.p;
+    px = dx.p;
   }
   const dim3 grid((unsigned)total);
+  const int ntasks = (int)tasks.size();
   auto launch = [=] {
-    auto go = [&](auto k) {
-      hipLaunchKernelGGL(k, grid, dim3(256), 0, s, pt, ps, pp);
+    auto go = [&](auto k, auto... more) {
+      hipLaunchKernelGGL(k, grid, dim3(256), 0, s, pt, ps, pp, more...);
       MXG_HIP(hipGetLastError());
     };
     if constexpr (std::is_same<T, float>::value)
-      if (bf16) return go(k_bgemm_bf16);
+      if (bf16) return runs ? go(k_bgemm_bf16<true>, px, ntasks) : go(k_bgemm_bf16<false>, px, ntasks);
     // slabs of 32 rows where a short FP32 tile's products would not cover its
     // loads (the FP32 sums over segments with 1 and 2 blocks: 25.0 and 28.1 us
     // against 29.0 and 33.1 with 16); in FP64 they gain nothing

@@ -53,3 +53,19 @@ def test_tile_heights(ctx, prec, m, n):
 def test_long_strides(ctx, prec, lda):
     check(ctx, prec, 0, 0, 130, 70, 5, 0.5, lda)
     check(ctx, prec, 1, 0, 66, 70, 18, 0., lda)
+
+
+@pytest.mark.parametrize("m,n", [(512, 512), (513, 511), (65, 4097), (2047, 2046), (2049, 1985)])  # 64 to 1056 tiles
+def test_bf16_tile_orders(ctx, m, n):
+    """bfloat16 products of few tiles (runs on an XCD) and of many (launch order), integers: exact."""
+    rng = np.random.default_rng(m)
+    for ta, tb, k in ((0, 0, 33), (1, 1, 16)):
+        A = rng.integers(-8, 9, (k, m) if ta else (m, k)).astype(np.float32)
+        B = rng.integers(-8, 9, (n, k) if tb else (k, n)).astype(np.float32)
+        Cm = rng.integers(-8, 9, (m, n)).astype(np.float32)
+        dA, dB, dC = padded(ctx, A, len(A) + 3), padded(ctx, B, len(B) + 5), padded(ctx, Cm, m + 2)
+        N.check_gpu(N.gpu().mxg_gemm(ctx.handle, N.MXG_BF16, ta, tb, m, n, k, 1.0, dA.ptr, len(A) + 3, dB.ptr, len(B) + 5,
+                                     2.0, dC.ptr, m + 2))
+        got = dC.download()
+        assert np.isnan(got[m:]).all()
+        assert np.array_equal(got[:m], (A.T if ta else A) @ (B.T if tb else B) + 2 * Cm)
