@@ -1034,7 +1034,17 @@ template void pair_jobs_append<float, bf16_t>(std::vector<PairJob>&, const std::
 void pair_list_upload(PairList& pl, const std::vector<PairJob>& jobs, hipStream_t s, bool few) {
   MXG_REQUIRE(jobs.size() < (1ull << 31), "pair list too long");
   pl.few = few;
-  for (const PairJob& j : jobs) pl.few = pl.few && !j.mx && j.n <= LAT_ROWS;
+  // Jobs of up to 32 x 32 entries are one wave's: all their loads are in flight at
+  // once there, too, and no barrier is needed (N = 65536, boxes of 32 at rank 16, FP32
+  // substitution of a vector on the sphere: 268 us with a workgroup each, 259 with a
+  // wave; 8 vectors 489 and 442; N = 4096, boxes of 128 at rank 32: 129 and 117). With
+  // 32 x 64 entries a workgroup is faster in FP64 (N = 9000, rank 64: 160 and 168).
+  bool small = true;
+  for (const PairJob& j : jobs) {
+    pl.few = pl.few && !j.mx && j.n <= LAT_ROWS;
+    small = small && (long long)j.n * j.m <= 1024;
+  }
+  pl.few = pl.few && !small;
   std::vector<PairJob> sorted;
   sorted.reserve(jobs.size());
   for (int mx : {1, 0}) {

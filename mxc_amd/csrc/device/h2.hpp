@@ -222,7 +222,8 @@ template <class T, class S>
 void pair_jobs_append(std::vector<PairJob>& jobs, const std::vector<PairTask>& tasks, const S* B, long long nB, const T* v,
                       long long nv, long long ldv, T* out, long long nout, long long ldo, bool matrix_cores = false);
 // few: the list comes from fewer than SPLIT_BELOW blocks, cut into chunks of
-// rows; it runs as one workgroup per job when no job has more than 64 rows
+// rows; it runs as one workgroup per job when no job has more than 64 rows and
+// some job more than 1024 entries
 void pair_list_upload(PairList& pl, const std::vector<PairJob>& jobs, hipStream_t s, bool few = false);
 // out[r + k ldo] = sum_c B[r + c*ld] v[c + k ldv] for every job and the
 // right-hand sides k < nrhs (<= MAX_RHS), one workgroup per job, blocks
