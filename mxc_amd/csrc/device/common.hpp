@@ -8,21 +8,15 @@
 #include <cstdint>
 #include <cstring>
 #include <functional>
-#include <map>
 #include <memory>
-#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
 
 #include "mxc_gpu.h"
+#include "pool.hpp"
 
 namespace mxg {
-
-struct Error : std::runtime_error {
-  int code;
-  Error(int c, const std::string& m) : std::runtime_error(m), code(c) {}
-};
 
 void set_last_error(const std::string& msg);
 // device address of the allocation-free dense check's scratch, looked up
@@ -58,63 +52,6 @@ int guarded(F&& f) {
     return MXG_ERR_ARG;
   }
 }
-
-// hipMalloc; when it fails, once more after every pool has given its kept blocks
-// back to the runtime.
-hipError_t device_malloc(void** p, size_t bytes);
-
-// Device memory of one context, kept for its later buffers: a factorization or a
-// level's construction allocates and frees 50 to 500 arrays, and hipFree alone
-// (which waits for the device) took 13 of the 54 ms of a preconditioner set-up
-// at N = 32768 and 8 of the 22.5 ms of a factorization at N = 131072.
-//
-// Blocks go back to the context they came from and every use of them is ordered
-// by that context's stream, so a block may be handed out again while the kernels
-// that used it last are still queued. All pools of the process keep at most a
-// thirty-second of the device's memory between them; beyond that the blocks kept
-// longest go, whichever pool has them (with the newest ones going instead, what
-// an earlier, larger object had left filled the pools for good: a factorization
-// at N = 131072 took 38 ms instead of 10 after ten other problems). Kept blocks
-// are given back when the context goes, and when any allocation of this library
-// fails.
-class DevPool {
- public:
-  explicit DevPool(int device);
-  ~DevPool();
-  DevPool(const DevPool&) = delete;
-  DevPool& operator=(const DevPool&) = delete;
-  // at least `bytes` bytes; *cap receives the block's size
-  void* take(size_t bytes, size_t* cap);
-  void give(void* p, size_t cap);
-  void trim();
-  // when its block kept longest came (the largest number if it has none), and that block's end
-  unsigned long long oldest();
-  void evict_oldest();
-  // bytes kept for reuse by the pools of a device
-  static size_t kept_on(int device);
-  // the pool the calling thread's buffers come from (set by PoolScope)
-  static std::shared_ptr<DevPool>& current();
-
- private:
-  int device_;
-  size_t kept_ = 0;
-  std::mutex mu_;
-  struct Block {
-    void* p;
-    unsigned long long age;
-  };
-  std::multimap<size_t, Block> free_;
-  std::map<unsigned long long, std::multimap<size_t, Block>::iterator> by_age_;
-};
-
-// Buffers allocated by this thread within the scope come from the pool.
-struct PoolScope {
-  std::shared_ptr<DevPool> before;
-  explicit PoolScope(const std::shared_ptr<DevPool>& p) : before(DevPool::current()) { DevPool::current() = p; }
-  ~PoolScope() { DevPool::current() = before; }
-  PoolScope(const PoolScope&) = delete;
-  PoolScope& operator=(const PoolScope&) = delete;
-};
 
 // Owning device buffer.
 template <class T>

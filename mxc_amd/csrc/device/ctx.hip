@@ -1,9 +1,6 @@
 // Context, memory helpers and error reporting of the device layer.
 // Replaces gpu_handles.cu:5-12 (device selection) and :54-71 (streams and
 // handles); there are no BLAS/SPARSE handles: every kernel is our own.
-#include <algorithm>
-#include <atomic>
-
 #include "common.hpp"
 
 namespace mxg {
@@ -11,157 +8,6 @@ namespace {
 thread_local std::string g_last_error;
 }
 void set_last_error(const std::string& msg) { g_last_error = msg; }
-
-// ---- device memory pools ----
-namespace {
-struct Pools {
-  std::mutex mu;  // taken before a pool's own
-  std::vector<DevPool*> all;
-  std::atomic<size_t> kept{0};  // bytes kept by all pools
-  std::atomic<size_t> most{0};  // and at most
-  std::atomic<unsigned long long> age{0};
-};
-// never destroyed: buffers may be released while the process ends
-Pools& pools() {
-  static Pools* p = new Pools;
-  return *p;
-}
-void trim_pools() {
-  Pools& P = pools();
-  std::lock_guard<std::mutex> lk(P.mu);
-  for (DevPool* p : P.all) p->trim();
-}
-}  // namespace
-
-hipError_t device_malloc(void** p, size_t bytes) {
-  hipError_t e = hipMalloc(p, bytes);
-  if (e != hipSuccess && pools().kept.load() > 0) {
-    (void)hipGetLastError();
-    trim_pools();
-    e = hipMalloc(p, bytes);
-  }
-  return e;
-}
-
-DevPool::DevPool(int device) : device_(device) {
-  size_t free_b = 0, total = 0;
-  if (hipMemGetInfo(&free_b, &total) != hipSuccess) total = 0;
-  Pools& P = pools();
-  std::lock_guard<std::mutex> lk(P.mu);
-  P.most = total / 32;
-  P.all.push_back(this);
-}
-
-DevPool::~DevPool() {
-  Pools& P = pools();
-  {
-    std::lock_guard<std::mutex> lk(P.mu);
-    P.all.erase(std::find(P.all.begin(), P.all.end(), this));
-  }
-  trim();
-}
-
-void* DevPool::take(size_t bytes, size_t* cap) {
-  // whole 512 bytes, above a megabyte whole 64 KB: arrays whose sizes differ
-  // little from one object to the next share blocks
-  const size_t unit = bytes > (size_t(1) << 20) ? size_t(65536) : size_t(512);
-  const size_t need = (bytes + unit - 1) / unit * unit;
-  {
-    std::lock_guard<std::mutex> lk(mu_);
-    auto it = free_.lower_bound(need);
-    if (it != free_.end() && it->first <= need + need / 4 + 4096) {
-      void* p = it->second.p;
-      by_age_.erase(it->second.age);
-      *cap = it->first;
-      kept_ -= it->first;
-      pools().kept -= it->first;
-      free_.erase(it);
-      return p;
-    }
-  }
-  void* p = nullptr;
-  const hipError_t e = device_malloc(&p, need);
-  if (e != hipSuccess)
-    throw Error(MXG_ERR_NOMEM, "hipMalloc of " + std::to_string(need) + " bytes failed: " + hipGetErrorString(e));
-  *cap = need;
-  return p;
-}
-
-void DevPool::give(void* p, size_t cap) {
-  Pools& P = pools();
-  if (cap > P.most.load()) {
-    (void)hipFree(p);
-    return;
-  }
-  {
-    std::lock_guard<std::mutex> lk(mu_);
-    const unsigned long long age = P.age++;
-    by_age_[age] = free_.emplace(cap, Block{p, age});
-    kept_ += cap;
-    P.kept += cap;
-  }
-  if (P.kept.load() <= P.most.load()) return;
-  std::lock_guard<std::mutex> lk(P.mu);
-  while (P.kept.load() > P.most.load()) {
-    DevPool* from = nullptr;
-    unsigned long long first = ~0ull;
-    for (DevPool* q : P.all) {
-      const unsigned long long a = q->oldest();
-      if (a < first) {
-        first = a;
-        from = q;
-      }
-    }
-    if (!from) break;
-    from->evict_oldest();
-  }
-}
-
-unsigned long long DevPool::oldest() {
-  std::lock_guard<std::mutex> lk(mu_);
-  return by_age_.empty() ? ~0ull : by_age_.begin()->first;
-}
-
-void DevPool::evict_oldest() {
-  void* p = nullptr;
-  {
-    std::lock_guard<std::mutex> lk(mu_);
-    if (by_age_.empty()) return;
-    const auto it = by_age_.begin()->second;
-    p = it->second.p;
-    kept_ -= it->first;
-    pools().kept -= it->first;
-    by_age_.erase(by_age_.begin());
-    free_.erase(it);
-  }
-  (void)hipFree(p);
-}
-
-void DevPool::trim() {
-  std::lock_guard<std::mutex> lk(mu_);
-  for (auto& b : free_) (void)hipFree(b.second.p);
-  pools().kept -= kept_;
-  kept_ = 0;
-  free_.clear();
-  by_age_.clear();
-}
-
-size_t DevPool::kept_on(int device) {
-  Pools& P = pools();
-  std::lock_guard<std::mutex> lk(P.mu);
-  size_t sum = 0;
-  for (DevPool* p : P.all)
-    if (p->device_ == device) {
-      std::lock_guard<std::mutex> lp(p->mu_);
-      sum += p->kept_;
-    }
-  return sum;
-}
-
-std::shared_ptr<DevPool>& DevPool::current() {
-  static thread_local std::shared_ptr<DevPool> p;
-  return p;
-}
 
 namespace {
 hipEvent_t take_event(mxg_ctx_s* c) {
