@@ -7,7 +7,7 @@
 
 namespace mxg {
 
-// What all pools keep, oldest first.
+// What all pools keep, device by device, oldest first.
 struct KeptBlocks {
   typedef std::multimap<size_t, DevPool::Block> Sizes;
   struct Device {
@@ -15,8 +15,7 @@ struct KeptBlocks {
     std::map<unsigned long long, std::pair<DevPool*, Sizes::iterator>> by_age;
   };
   std::mutex mu;
-  Device all;
-  std::map<int, size_t> bytes_on;  // of a device's pools
+  std::map<int, Device> devices;
   unsigned long long age = 0;
 
   // never destroyed: buffers may be released while the process ends
@@ -28,7 +27,7 @@ struct KeptBlocks {
   // The rest with the lock held.
 
   void keep(DevPool* pool, void* p, size_t cap) {
-    Device& d = all;
+    Device& d = devices[pool->device_];
     const unsigned long long a = age++;
     const auto it = pool->free_.emplace(cap, DevPool::Block{p, a});
     try {
@@ -38,13 +37,11 @@ struct KeptBlocks {
       throw;
     }
     d.bytes += cap;
-    bytes_on[pool->device_] += cap;
   }
   void* drop(DevPool* pool, Sizes::iterator it) {
-    Device& d = all;
+    Device& d = devices[pool->device_];
     void* p = it->second.p;
     d.bytes -= it->first;
-    bytes_on[pool->device_] -= it->first;
     d.by_age.erase(it->second.age);
     pool->free_.erase(it);
     return p;
@@ -76,8 +73,13 @@ void free_while(Next next) {
 hipError_t device_malloc(void** p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
   if (e == hipSuccess) return e;
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess || DevPool::kept_on(device) == 0) return e;
   (void)hipGetLastError();
-  free_while([](KeptBlocks& K) -> void* { return K.all.by_age.empty() ? nullptr : K.drop_oldest(K.all); });
+  free_while([device](KeptBlocks& K) -> void* {
+    KeptBlocks::Device& d = K.devices[device];
+    return d.by_age.empty() ? nullptr : K.drop_oldest(d);
+  });
   return hipMalloc(p, bytes);
 }
 
@@ -86,7 +88,7 @@ DevPool::DevPool(int device) : device_(device) {
   if (hipMemGetInfo(&free_b, &total) != hipSuccess) total = 0;
   KeptBlocks& K = KeptBlocks::get();
   std::lock_guard<std::mutex> lk(K.mu);
-  K.all.most = total / 32;
+  K.devices[device].most = total / 32;
 }
 
 DevPool::~DevPool() {
@@ -120,7 +122,7 @@ void DevPool::give(void* p, size_t cap) noexcept {
   try {
     KeptBlocks& K = KeptBlocks::get();
     std::lock_guard<std::mutex> lk(K.mu);
-    if (cap <= K.all.most) {
+    if (cap <= K.devices[device_].most) {
       K.keep(this, p, cap);
       kept = true;
     }
@@ -130,13 +132,17 @@ void DevPool::give(void* p, size_t cap) noexcept {
     (void)hipFree(p);
     return;
   }
-  free_while([](KeptBlocks& K) -> void* { return K.all.bytes > K.all.most ? K.drop_oldest(K.all) : nullptr; });
+  free_while([this](KeptBlocks& K) -> void* {
+    KeptBlocks::Device& d = K.devices[device_];
+    return d.bytes > d.most ? K.drop_oldest(d) : nullptr;
+  });
 }
 
 size_t DevPool::kept_on(int device) {
   KeptBlocks& K = KeptBlocks::get();
   std::lock_guard<std::mutex> lk(K.mu);
-  return K.bytes_on[device];
+  const auto it = K.devices.find(device);
+  return it == K.devices.end() ? 0 : it->second.bytes;
 }
 
 std::shared_ptr<DevPool>& DevPool::current() {

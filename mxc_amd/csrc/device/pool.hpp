@@ -18,8 +18,8 @@ struct Error : std::runtime_error {
   Error(int c, const std::string& m) : std::runtime_error(m), code(c) {}
 };
 
-// hipMalloc; when it fails, once more after every pool has given its kept blocks
-// back to the runtime.
+// hipMalloc on the current device; when it fails, once more after the device's
+// pools have given their kept blocks back to the runtime.
 hipError_t device_malloc(void** p, size_t bytes);
 
 // A factorization or a level's construction allocates and frees 50 to 500 arrays,
@@ -29,12 +29,12 @@ hipError_t device_malloc(void** p, size_t bytes);
 //
 // Blocks go back to the context they came from and every use of them is ordered
 // by that context's stream, so a block may be handed out again while the kernels
-// that used it last are still queued. All pools of the process keep at most a
-// thirty-second of the device's memory between them; beyond that the blocks kept
-// longest go, whichever pool has them (with the newest ones going instead, what an earlier,
+// that used it last are still queued. The pools of a device keep at most a
+// thirty-second of its memory between them; beyond that the blocks kept longest go,
+// whichever pool has them (with the newest ones going instead, what an earlier,
 // larger object had left filled the pools for good: a factorization at N = 131072
 // took 38 ms instead of 10 after ten other problems). Kept blocks are given back
-// when the context goes, and when any allocation of this library
+// when the context goes, and when any allocation of this library on the device
 // fails. hipFree is never called with a lock held: it waits for the device, and a
 // context that is being made or another thread's allocation would wait with it.
 class DevPool {

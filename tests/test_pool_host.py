@@ -7,7 +7,7 @@ import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 ROCM = os.environ.get("ROCM", "/opt/rocm")
-CASES = ["reuse", "oldest_go", "failing_allocation", "free_without_locks", "threads"]
+CASES = ["reuse", "oldest_go", "failing_allocation", "free_without_locks", "per_device", "threads"]
 
 
 def build(tmp, *flags):
