@@ -23,6 +23,10 @@
 // products.
 #include "h2.hpp"
 
+#include <optional>
+
+#include "fork.hpp"
+
 #include <algorithm>
 #include <numeric>
 
@@ -793,20 +797,20 @@ void h2_matvec_levels(mxg_h2_s* h, T* y, long long ldy, int nrhs) {
   // is bound by bytes, and beside the near products it would have the few CUs
   // left to the context stream (N = 131072, 8 right-hand sides: 79 us there, 21
   // alone)
+  std::optional<Fork> near;
   for (long long l = L; l >= 0; l--) {
     if (h->lv[l].lenZ > 0) {
       ProfScope prof(h->ctx, MXG_PROF_MATVEC_UPPER);
       pair_gemv<T, T>(h->lv[l].up_pl[pi], nrhs, s);
     }
     if (l == L) {
-      MXG_HIP(hipEventRecord(h->ctx->fork, s));
-      MXG_HIP(hipStreamWaitEvent(sa, h->ctx->fork, 0));
+      near.emplace(s, sa, h->ctx->fork, h->ctx->join);
       ProfScope prof(h->ctx, f64 ? MXG_PROF_MATVEC_LEAF_FP64 : MXG_PROF_MATVEC_LEAF_FP32, sa);
       // one of the two lists is empty
       sym_gemv<T>(h->near_sym[pi], nrhs, sa);
       pair_gemv<T, T>(h->near_pl[pi], nrhs, sa);
       prof.end();
-      MXG_HIP(hipEventRecord(h->ctx->join, sa));
+      near->done();
     }
   }
   // every far term of every level, one launch
@@ -820,7 +824,7 @@ void h2_matvec_levels(mxg_h2_s* h, T* y, long long ldy, int nrhs) {
   for (long long l = 0; l <= L; l++) {
     Level& Lv = h->lv[l];
     const bool leaf = (l == L);
-    if (leaf) MXG_HIP(hipStreamWaitEvent(s, h->ctx->join, 0));
+    if (leaf) near->wait();
     T* out = leaf ? y : Ops<T>::W(h, l + 1);
     const long long ldo = leaf ? ldy : h->lv[l + 1].lenZ;
     if (!leaf && ldo == 0) continue;

@@ -1,5 +1,6 @@
-// The device layer's memory pools (pool.cpp) against counting stand-ins for the
-// runtime's allocation calls: pool_host CASE exits 0 when the case holds.
+// The device layer's memory pools (pool.cpp) and stream forks (fork.hpp) against
+// counting stand-ins for the runtime's calls: pool_host CASE exits 0 when the case
+// holds.
 #include <atomic>
 #include <chrono>
 #include <condition_variable>
@@ -14,6 +15,7 @@
 #include <thread>
 #include <vector>
 
+#include "fork.hpp"
 #include "pool.hpp"
 
 using mxg::DevPool;
@@ -25,6 +27,7 @@ std::map<int, size_t> used;
 size_t capacity = size_t(1) << 40;             // of a device
 constexpr size_t TOTAL = size_t(1) << 20;      // the device memory that hipMemGetInfo reports: pools keep 32 KB
 thread_local int device = 0;
+std::string events;                            // the event calls so far
 std::function<void()> on_free;                 // called within hipFree
 
 void check(bool ok, const char* what) {
@@ -66,6 +69,14 @@ hipError_t hipMemGetInfo(size_t* f, size_t* t) {
 }
 hipError_t hipGetDevice(int* d) {
   *d = device;
+  return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+  events += "record " + std::to_string((size_t)e) + " on " + std::to_string((size_t)s) + ";";
+  return hipSuccess;
+}
+hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
+  events += std::to_string((size_t)s) + " waits for " + std::to_string((size_t)e) + ";";
   return hipSuccess;
 }
 hipError_t hipGetLastError() { return hipSuccess; }
@@ -220,13 +231,33 @@ void threads() {
   for (auto& t : ts) t.join();
   check(live.empty() && DevPool::kept_on(0) == 0 && DevPool::kept_on(1) == 0, "everything given back");
 }
+
+// The first stream (1) waits for the second (2) once, also when the work in between ends in an error.
+void forks() {
+  const auto first = (hipStream_t)1, second = (hipStream_t)2;
+  const auto fork = (hipEvent_t)3, join = (hipEvent_t)4;
+  const std::string begin = "record 3 on 1;2 waits for 3;", end = "record 4 on 2;1 waits for 4;";
+  for (int stop = 0; stop < 3; stop++) {  // at the second stream's work, after it, not at all
+    events.clear();
+    try {
+      mxg::Fork f(first, second, fork, join);
+      if (stop == 0) throw 0;
+      f.done();
+      if (stop == 1) throw 0;
+      f.wait();
+    } catch (int) {
+    }
+    check(events == begin + end, events.c_str());
+  }
+}
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::map<std::string, void (*)()> cases{{"reuse", reuse}, {"oldest_go", oldest_go},
                                                 {"failing_allocation", failing_allocation},
                                                 {"free_without_locks", free_without_locks},
-                                                {"per_device", per_device}, {"threads", threads}};
+                                                {"per_device", per_device}, {"threads", threads},
+                                                {"forks", forks}};
   check(argc == 2 && cases.count(argv[1]), "a case by name");
   cases.at(argv[1])();
   std::lock_guard<std::mutex> lk(mu);

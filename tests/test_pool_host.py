@@ -1,5 +1,6 @@
-"""The device memory pools' bookkeeping (pool.cpp) on the CPU: built with stand-ins
-for the runtime's allocation calls, and once more under the thread sanitizer."""
+"""The device memory pools' bookkeeping (pool.cpp) and the order of forked streams
+(fork.hpp) on the CPU: built with stand-ins for the runtime's calls, and the pools
+once more under the thread sanitizer."""
 import os
 import subprocess
 
@@ -7,7 +8,7 @@ import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 ROCM = os.environ.get("ROCM", "/opt/rocm")
-CASES = ["reuse", "oldest_go", "failing_allocation", "free_without_locks", "per_device", "threads"]
+CASES = ["reuse", "oldest_go", "failing_allocation", "free_without_locks", "per_device", "threads", "forks"]
 
 
 def build(tmp, *flags):
