@@ -67,12 +67,13 @@ __device__ inline unsigned long long sketch_word(unsigned long long t, unsigned 
 
 // Omega as signed bytes in the order the matrix cores take it: 16 rows (group
 // g) x 64 far rows (block u) are 1024 contiguous bytes, lane 16 k + r holding
-// rows r and far rows 64 u + 16 k .. + 15. One thread per 16 bytes.
-__global__ void __launch_bounds__(256) k_sketch_signs(u4* __restrict__ signs, int nu) {
+// rows r and far rows 64 u + 16 k .. + 15; the table holds nu blocks from block u0
+// on. One thread per 16 bytes.
+__global__ void __launch_bounds__(256) k_sketch_signs(u4* __restrict__ signs, int nu, int u0) {
   const long long e = (long long)blockIdx.x * 256 + threadIdx.x;  // u, then lane
   if (e >= 64ll * nu) return;
   const int g = blockIdx.y, lane = (int)(e & 63), row = 16 * g + (lane & 15);
-  const long long t0 = (e >> 6) * 64 + 16 * (lane >> 4);
+  const long long t0 = (u0 + (e >> 6)) * 64 + 16 * (lane >> 4);
   u4 v;
 #pragma unroll
   for (int q = 0; q < 4; q++) {
@@ -107,7 +108,7 @@ __device__ inline void bytes_of(unsigned a, unsigned b, unsigned c, unsigned d, 
 // 16 x 16; KT far rows per step.
 template <int KID, int WR, int RW, int CT, int KT>
 __global__ void __launch_bounds__(512) k_sketch(const SketchTask* __restrict__ tasks, const double* __restrict__ bodies,
-                                                EvalArgs ke, const u4* __restrict__ signs, int nu) {
+                                                EvalArgs ke, const u4* __restrict__ signs, int nu, int u0) {
   constexpr int WC = 8 / WR, TC = 16 * CT * WC;
   constexpr int E = KT * TC / 512;  // entries a thread evaluates per step: consecutive rows of one column
   constexpr int SUB = 16 / E;       // threads sharing 16 rows of a column
@@ -252,7 +253,7 @@ __global__ void __launch_bounds__(512) k_sketch(const SketchTask* __restrict__ t
   auto row_coord = [&](int idx) { return idx >= 0 ? bodies[3 * (long long)idx + xc] : 0.; };
   const int wr = wave % WR, wc = wave / WR;
   const int g0 = (tk.i0 >> 4) + wr * RW;  // first row group (16 rows) of the wave
-  const u4* sg = signs + 64ll * nu * g0 + lane;
+  const u4* sg = signs + 64ll * ((long long)nu * g0 - u0) + lane;
   constexpr bool AHEAD = RW * KT <= 128;  // signs loaded one step ahead, where registers allow it
   i4 om[AHEAD ? RW : 1];
   auto load_signs = [&](int i, int tb) { return *reinterpret_cast<const i4*>(sg + 64ll * (nu * i + (tb >> 6))); };
@@ -402,6 +403,7 @@ __global__ void __launch_bounds__(256) k_sum_slices(const SliceSum* __restrict__
 struct SketchShape {
   int rows, cols;
 };
+constexpr size_t SIGNS_BYTES = 64 << 20;  // of the sign table
 constexpr SketchShape SKETCH_SHAPES[] = {{64, 64}, {128, 64}, {256, 32}, {384, 32}, {512, 16}};
 int sketch_shape(int M) {
   int k = 0;
@@ -411,15 +413,15 @@ int sketch_shape(int M) {
 
 template <int KID>
 void launch_sketch(int shape, unsigned grid, const SketchTask* tasks, const double* bodies, mxg_kernel_t k,
-                   const u4* signs, int nu, hipStream_t s) {
+                   const u4* signs, int nu, int u0, hipStream_t s) {
   const dim3 g(grid), blk(512);
   const EvalArgs ke = eval_args(k);
   switch (shape) {
-    case 0: hipLaunchKernelGGL((k_sketch<KID, 4, 1, 2, 64>), g, blk, 0, s, tasks, bodies, ke, signs, nu); break;
-    case 1: hipLaunchKernelGGL((k_sketch<KID, 8, 1, 4, 64>), g, blk, 0, s, tasks, bodies, ke, signs, nu); break;
-    case 2: hipLaunchKernelGGL((k_sketch<KID, 8, 2, 2, 64>), g, blk, 0, s, tasks, bodies, ke, signs, nu); break;
-    case 3: hipLaunchKernelGGL((k_sketch<KID, 8, 3, 2, 64>), g, blk, 0, s, tasks, bodies, ke, signs, nu); break;
-    default: hipLaunchKernelGGL((k_sketch<KID, 8, 4, 1, 128>), g, blk, 0, s, tasks, bodies, ke, signs, nu); break;
+    case 0: hipLaunchKernelGGL((k_sketch<KID, 4, 1, 2, 64>), g, blk, 0, s, tasks, bodies, ke, signs, nu, u0); break;
+    case 1: hipLaunchKernelGGL((k_sketch<KID, 8, 1, 4, 64>), g, blk, 0, s, tasks, bodies, ke, signs, nu, u0); break;
+    case 2: hipLaunchKernelGGL((k_sketch<KID, 8, 2, 2, 64>), g, blk, 0, s, tasks, bodies, ke, signs, nu, u0); break;
+    case 3: hipLaunchKernelGGL((k_sketch<KID, 8, 3, 2, 64>), g, blk, 0, s, tasks, bodies, ke, signs, nu, u0); break;
+    default: hipLaunchKernelGGL((k_sketch<KID, 8, 4, 1, 128>), g, blk, 0, s, tasks, bodies, ke, signs, nu, u0); break;
   }
   MXG_HIP(hipGetLastError());
 }
@@ -428,17 +430,26 @@ void launch_sketch(int shape, unsigned grid, const SketchTask* tasks, const doub
 
 void sketch_rows(mxg_ctx_s* ctx, const std::vector<SketchBox>& boxes, const double* d_bodies, mxg_kernel_t k,
                  double* d_partial, hipStream_t s) {
-  std::map<int, std::vector<SketchTask>> tasks;  // by tile shape
+  long long maxM = 0, maxnf = 0;
+  for (const SketchBox& b : boxes) {
+    if (b.M <= 0 || b.nf <= 0) continue;
+    maxM = std::max<long long>(maxM, b.M);
+    maxnf = std::max(maxnf, b.nf);
+  }
+  MXG_REQUIRE(maxnf < (1ll << 31), "far list too long");
+  // The signs of every row group a tile can cover (up to 512 rows a tile), for
+  // whole slices of far rows. Longer lists than SIGNS_BYTES have room for, 131072
+  // rows with boxes of up to 512 columns, take turns in the table.
+  const unsigned groups = (unsigned)((maxM + 511) / 512 * 32);
+  const long long window = std::max<long long>(SIGNS_BYTES / (16 * std::max(groups, 1u)) / SKETCH_ROWS, 1) * SKETCH_ROWS;
+  std::map<std::pair<long long, int>, std::vector<SketchTask>> tasks;  // by window and tile shape
   std::vector<SliceSum> sums;
   std::vector<long long> prefix{0};
   size_t poff = 0;
   double flops = 0.;
-  long long maxM = 0, maxnf = 0;
   for (const SketchBox& b : boxes) {
     if (b.M <= 0 || b.nf <= 0) continue;
     flops += 2. * b.M * (double)b.M * (double)b.nf;
-    maxM = std::max<long long>(maxM, b.M);
-    maxnf = std::max(maxnf, b.nf);
     const int nsplit = (int)((b.nf + SKETCH_ROWS - 1) / SKETCH_ROWS);
     const long long len = (long long)b.M * b.M;
     double* base = nsplit == 1 ? b.Y : d_partial + poff;
@@ -447,7 +458,7 @@ void sketch_rows(mxg_ctx_s* ctx, const std::vector<SketchBox>& boxes, const doub
       const int t0 = sp * SKETCH_ROWS, t1 = (int)std::min<long long>(b.nf, (long long)(sp + 1) * SKETCH_ROWS);
       for (int i0 = 0; i0 < b.M; i0 += SKETCH_SHAPES[shape].rows)
         for (int j0 = 0; j0 < b.M; j0 += SKETCH_SHAPES[shape].cols)
-          tasks[shape].push_back(SketchTask{b.rows, b.cols, base + sp * len, t0, t1, b.M, i0, j0, 0});
+          tasks[{t0 / window, shape}].push_back(SketchTask{b.rows, b.cols, base + sp * len, t0, t1, b.M, i0, j0, 0});
     }
     if (nsplit > 1) {
       sums.push_back(SliceSum{base, b.Y, len, nsplit, 0});
@@ -462,23 +473,25 @@ void sketch_rows(mxg_ctx_s* ctx, const std::vector<SketchBox>& boxes, const doub
     MXG_REQUIRE(kv.second.size() < (1u << 31), "sketch grid too large");
     dts[q++].upload(kv.second, s);
   }
-  // signs of every row group a tile can cover (up to 512 rows a tile) and of
-  // whole steps of 128 far rows
-  const long long nu = (maxnf + 127) / 128 * 2;
-  const unsigned groups = (unsigned)((maxM + 511) / 512 * 32);
-  MXG_REQUIRE(64 * nu < (1ll << 31), "far list too long");
+  const long long nu = (std::min(maxnf, window) + 127) / 128 * 2;  // whole steps of 128 far rows
   DevBuf<u4> signs;
   signs.alloc((size_t)(64 * nu) * groups);
   ProfScope prof(ctx, MXG_PROF_SKETCH, s, flops);
-  hipLaunchKernelGGL(k_sketch_signs, dim3(ceil_div(64 * nu, 256), groups), dim3(256), 0, s, signs.p, (int)nu);
-  MXG_HIP(hipGetLastError());
   q = 0;
+  long long filled = -1;
   for (const auto& kv : tasks) {
+    const int u0 = (int)(kv.first.first * window / 64);
+    if (kv.first.first != filled) {
+      hipLaunchKernelGGL(k_sketch_signs, dim3(ceil_div(64 * nu, 256), groups), dim3(256), 0, s, signs.p, (int)nu, u0);
+      MXG_HIP(hipGetLastError());
+      filled = kv.first.first;
+    }
     const unsigned g = (unsigned)kv.second.size();
     const SketchTask* tp = dts[q++].p;
-    if (k.id == MXG_KERNEL_GAUSSIAN) launch_sketch<MXG_KERNEL_GAUSSIAN>(kv.first, g, tp, d_bodies, k, signs.p, (int)nu, s);
-    else if (k.id == MXG_KERNEL_YUKAWA) launch_sketch<MXG_KERNEL_YUKAWA>(kv.first, g, tp, d_bodies, k, signs.p, (int)nu, s);
-    else launch_sketch<MXG_KERNEL_LAPLACE>(kv.first, g, tp, d_bodies, k, signs.p, (int)nu, s);
+    const int shape = kv.first.second;
+    if (k.id == MXG_KERNEL_GAUSSIAN) launch_sketch<MXG_KERNEL_GAUSSIAN>(shape, g, tp, d_bodies, k, signs.p, (int)nu, u0, s);
+    else if (k.id == MXG_KERNEL_YUKAWA) launch_sketch<MXG_KERNEL_YUKAWA>(shape, g, tp, d_bodies, k, signs.p, (int)nu, u0, s);
+    else launch_sketch<MXG_KERNEL_LAPLACE>(shape, g, tp, d_bodies, k, signs.p, (int)nu, u0, s);
   }
   DevBuf<SliceSum> ds;
   DevBuf<long long> dp;

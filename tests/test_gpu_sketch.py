@@ -5,6 +5,7 @@ import ctypes as C
 
 import numpy as np
 import pytest
+import scipy.linalg
 
 import oracle_lib as O
 from mxc_amd import _native as N
@@ -138,3 +139,56 @@ def test_columns_that_are_not_finite(ctx, M, case):
     pts[col] = np.nan if case == "overflow" else 1e160
     r0, q0 = first_basis(ctx, pts, M, far, kernel, 1e3, alpha)
     assert r == r0 and np.abs(q[rest] - q0[rest]).max() < 1e-9
+
+
+def signs(t, i):
+    """The sketch's sign of far row t and row i: bit i % 64 of a 64-bit hash of (t, i / 64)."""
+    with np.errstate(over="ignore"):
+        z = (t[None, :] * np.uint64(0x9E3779B97F4A7C15) + (i >> np.uint64(6))[:, None] * np.uint64(0xD1B54A32D192ED03)
+             + np.uint64(0x632BE59BD9B4E019))
+        z = (z ^ (z >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+        z = (z ^ (z >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+        z ^= z >> np.uint64(31)
+    return 1.0 - 2.0 * ((z >> (i & np.uint64(63))[:, None]) & np.uint64(1)).astype(np.float64)
+
+
+@pytest.mark.parametrize("M,nf", [(40, 131072 - 70), (40, 131072 + 70), (70, 2 * 131072 + 8192 + 1), (1030, 5 * 8192 + 3)])
+def test_long_far_lists(ctx, M, nf):
+    """Lists of more far rows than the table of signs holds at a time, against the same sketch in numpy."""
+    rows = 900
+    pts = apart(M, rows, 28)
+    far = M + np.arange(nf) * 7 % rows  # every row again and again
+    r, q = first_basis(ctx, pts, M, far, "laplace")
+    per_row = np.zeros((M, rows))  # the signs of each body's rows, summed
+    for a in range(0, nf, 8192):
+        t = np.arange(a, min(a + 8192, nf))
+        s = signs(t.astype(np.uint64), np.arange(M, dtype=np.uint64))
+        for b in range(rows):
+            per_row[:, b] += s[:, far[t] - M == b].sum(1)
+    G = 1.0 / np.sqrt(((pts[M:, None, :] - pts[None, :M, :]) ** 2).sum(-1))
+    _, R, piv = scipy.linalg.qr(per_row @ G, mode="economic", pivoting=True)
+    d = np.abs(np.diag(R))
+    k = int((d > 1e-2 * d.max()).sum())
+    assert 0 < k < M and r == k
+    ref = np.zeros((M, k))
+    ref[piv[:k]] = np.eye(k)
+    ref[piv[k:]] = np.linalg.solve(R[:k, :k], R[:k, k:]).T
+    # the same pivots: rounding, amplified by the conditioning of the kept columns, about 100
+    assert np.abs(q[:, :k] - ref).max() < 1e4 * M * 2.0**-52
+
+
+def test_memory_of_long_far_lists(ctx):
+    """The table of signs stays small beside the list itself."""
+    hip = C.CDLL("libamdhip64.so")
+
+    def free():
+        f, t = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+    M, rows, nf = 40, 900, 4 << 20
+    pts = apart(M, rows, 29)
+    first_basis(ctx, pts, M, M + np.arange(9000) % rows, "laplace")
+    before = free()
+    first_basis(ctx, pts, M, M + np.arange(nf) % rows, "laplace")
+    # the list (4 bytes an entry), the table (64 MB) and slices, all kept by the context's pool at most
+    assert before - free() < 4 * nf + (96 << 20)
