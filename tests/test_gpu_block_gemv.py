@@ -79,3 +79,24 @@ def test_block_product_rejects_bad_arguments(ctx):
     assert G.mxg_block_gemv(ctx.handle, N.MXG_FP64, 4, 4, one.ptr, 4, one.ptr, 4, one.ptr, 4, 9, 0) == N.MXG_ERR_ARG
     assert G.mxg_block_gemv(ctx.handle, 7, 4, 4, one.ptr, 4, one.ptr, 4, one.ptr, 4, 1, 0) == N.MXG_ERR_ARG
     one.free()
+
+
+@pytest.mark.timeout(120)
+@pytest.mark.parametrize("n,m,ldb", [(1, 7, 4), (63, 33, 64), (93, 94, 96), (193, 130, 196), (257, 40, 260), (301, 512, 304)])
+@pytest.mark.parametrize("storage", ["bf16", "fp32", "fp64"])
+@pytest.mark.parametrize("units", [0, 1], ids=["vector", "matrix"])
+def test_ragged_rows_of_aligned_columns(ctx, n, m, ldb, storage, units):
+    """Rows that are no multiple of a vector load's, in columns that are aligned: the loads reach into the padding rows
+    (NaN here), whose products are neither used nor written."""
+    rng = np.random.default_rng(n + m)
+    full = np.full((ldb, m), np.nan)
+    full[:n] = rng.integers(-8, 9, (n, m))  # small integers: exact in every storage
+    code = {"bf16": N.MXG_BF16, "fp32": N.MXG_FP32, "fp64": N.MXG_FP64}[storage]
+    dtype = np.float64 if storage == "fp64" else np.float32
+    st = to_bf16(full) if storage == "bf16" else full.astype(dtype)
+    for nrhs in (1, 2, 3, 8):
+        X = np.asfortranarray(rng.integers(-8, 9, (m, nrhs)).astype(dtype))
+        dB, dX, dY = ctx.array(np.asfortranarray(st)), ctx.array(X), ctx.array(np.full((n + 5, nrhs), 77, dtype, order="F"))
+        N.check_gpu(N.gpu().mxg_block_gemv(ctx.handle, code, n, m, dB.ptr, ldb, dX.ptr, m, dY.ptr, n + 5, nrhs, units))
+        Y = dY.download()
+        assert np.array_equal(Y[:n], full[:n] @ X) and (Y[n:] == 77).all(), nrhs
