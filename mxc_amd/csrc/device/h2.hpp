@@ -129,8 +129,9 @@ struct Level {
   // (offsets offC32), so that its columns admit 16-byte loads.
   DevBuf<float> A32, Q32, C32;
   std::vector<long long> offC32;
-  // matvec tasks: up z_i = QT_i x_i (QT_i = Q_i[:, :k]^T, k x M), far
-  // t_p = C_p z_j, leaf near u_p = A_p x_j; toffF / toffN: term offsets
+  // matvec tasks: up z_i = QT_i x_i (QT_i = Q_i[:, :k]^T, k x M, its leading
+  // dimension k rounded up to 4), far t_p = C_p z_j, leaf near u_p = A_p x_j;
+  // toffF / toffN: term offsets
   // within the level's share of the term scratch (tbaseF / tbaseN; the FP32
   // far terms have the padded row counts of C32: far_t32, toffF32)
   std::vector<long long> offQT, toffF, toffN, toffF32;

@@ -47,7 +47,8 @@ inline EvalArgs eval_args(mxg_kernel_t k) {
                   std::sqrt(far2) * 0.288};
 }
 
-// 1 / sqrt(x) from the hardware's estimate and one step of third order.
+// 1 / sqrt(x) from the hardware's estimate y and the first terms of the binomial
+// series of (1 - e)^(-1/2), e = 1 - x y^2.
 __device__ inline double rsqrt_refined(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   const double e = fma(-x * y, y, 1.0);

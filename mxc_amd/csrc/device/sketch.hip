@@ -33,9 +33,9 @@
 // thread evaluates 4 or 8 entries of one column and writes their bytes to LDS
 // as the matrix cores read them, 16 rows of one byte and column side by side;
 // the buffers alternate, so a step has one barrier. The signs come as bytes from
-// a table filled once per call and shared by all boxes: making the bytes of a
-// wave's rows from sign bits in every step took a quarter of the vector
-// instructions.
+// a table shared by all boxes and filled once per call, or per window of a long
+// list's rows: making the bytes of a wave's rows from sign bits in every step took a
+// quarter of the vector instructions.
 //
 // Measured on the operator of the unit sphere at N = 65536 (eps 1e-12, boxes of
 // 256 to 350 columns, 3.7e12 flops): 95.6 ms on the FP64 matrix cores, 28.9 ms

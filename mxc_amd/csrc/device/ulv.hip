@@ -207,14 +207,16 @@ struct UlvImpl : UlvBase {
     // substitution task lists: x = V y per box; sr terms A_ij[:s_i, s_j:] x_j[s_j:]
     // (forward) and rs terms A_ij[s_i:, :s_j] w_j (backward) per near pair
     PairList v_pl, fwd_pl, bwd_pl;
-    // leaf only: y_i = U_i v_i over the gathered backward vectors (ubuf)
+    // leaf only: y_i = U_i v_i over its gathered backward vectors (ubuf)
     PairList u_pl;
     DevBuf<long long> d_toffU, d_toffB;
     bool vecM = false;
   };
   std::vector<Lv> lv;
   DevBuf<T> vin, tbuf;  // n and tlen entries per right-hand side
-  DevBuf<T> ubuf;       // the leaf's backward vectors [w_i ; x_i[s:] - sum t], n per right-hand side
+  // a level's backward vectors [w_i ; x_i[s:] - sum t], n per right-hand side: the
+  // leaf's, and for groups of 4 and 8 those of levels with few boxes
+  DevBuf<T> ubuf;
   long long tlen = 1;
 
   explicit UlvImpl(mxg_h2_s* hh, bool sbf16 = false) : h(hh), schur_bf16(sbf16) {
